@@ -300,13 +300,20 @@ int mr_gemm(int layout, int64_t M, int64_t N, int64_t K, const void* A, int64_t 
             void* stream);
 
 /*
- * fp32 GEMM on the MFMA cores (fp32 products and accumulation), any sizes:
+ * fp32 GEMM on the MFMA cores (float32's precision and range: operands in
+ * three exact bf16 planes, fp32 accumulation), any sizes:
  *   C[m, n] = sum_k A(m, k) (B(n, k) - B2(n, k))   (B2 may be NULL)
  * in the layouts of mr_gemm (B2 shares B's layout and ldb); C fp32 [M, N]
  * row-major. Replaces the float32 products of the reference's single-layer
  * loop, the layer residual x (W' - W)^T and the weight gradient
- * (dL/dr)^T x (mround/core/tuning.py:140-190).
+ * (dL/dr)^T x (mround/core/tuning.py:140-190). The _ws form takes a workspace
+ * for the k-split partials of a grid that would leave CUs idle (16-byte
+ * aligned; a smaller or NULL one drops the split).
  */
+size_t mr_gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int mr_gemm_f32_ws(int layout, int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, const float* B,
+                   const float* B2, int64_t ldb, float* C, int64_t ldc, void* workspace,
+                   size_t workspace_bytes, void* stream);
 int mr_gemm_f32(int layout, int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, const float* B,
                 const float* B2, int64_t ldb, float* C, int64_t ldc, void* stream);
 

@@ -10,7 +10,7 @@ it: the residual then carries only its own rounding, not that of two large
 products subtracted.
 
 Per step: W' by the fake-quant kernel (fp32), the residual and dL/dW' as two
-fp32 MFMA GEMMs (``mr_gemm_f32``: ``x (W' - W)^T``, the difference formed as
+GEMMs to float32's precision (``mr_gemm_f32``: ``x (W' - W)^T``, the difference formed as
 the operand is loaded, and ``(dL/dr)^T x``, any shape), the loss and dL/dr
 by the loss kernels (the outlier rule's threshold on the device), and the
 straight-through gradient, sign step and projection in one fused kernel on

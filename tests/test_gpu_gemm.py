@@ -369,3 +369,62 @@ def test_gemm_f32(layout, mnk, minus):
     c2 = torch.empty(M, N, device=dev())
     K.gemm_f32(layout, A.to(dev()), B.to(dev()), c2, M=M, N=N, K=Kd, b_minus=None if B2 is None else B2.to(dev()))
     assert torch.equal(c2.cpu(), c[:M, :N].cpu())
+
+
+# The k-split grids, vector and element loads (odd leading dimensions), against
+# float64 within the same bound; without a workspace the whole-K sum agrees to it.
+@pytest.mark.parametrize("layout", ["nt", "nn", "tn"])
+@pytest.mark.parametrize("mnk", [(256, 128, 4096), (130, 258, 3001), (896, 1000, 1024), (129, 64, 160)])
+@pytest.mark.parametrize("pad", [0, 1, 4])
+def test_gemm_f32_split(layout, mnk, pad):
+    M, N, Kd = mnk
+    print("case gemm f32 split", layout, mnk, pad, flush=True, file=sys.stderr)
+    g = torch.Generator().manual_seed(M + pad)
+    a, b, b2 = (torch.randn(r, Kd, generator=g) * 10.0 ** (4 * torch.rand(r, 1, generator=g) - 2) for r in (M, N, N))
+    b2 = b * (1 + 1e-3 * b2)  # B - B2 loses most of B's bits, as W' - W does
+    want = a.double() @ (b - b2).double().T
+    bound = (Kd + 4) * 2.0**-23 * (a.double().abs() @ (b - b2).double().abs().T)
+
+    def lay(t, kmajor):
+        t = t if kmajor else t.T.contiguous()
+        buf = torch.full((t.shape[0], t.shape[1] + pad), float("nan"))
+        buf[:, :t.shape[1]] = t
+        return buf.to(dev())[:, :t.shape[1]]
+
+    A, B, B2 = lay(a, layout != "tn"), lay(b, layout == "nt"), lay(b2, layout == "nt")
+    c = torch.empty(M, N, device=dev())
+    K.gemm_f32(layout, A, B, c, M=M, N=N, K=Kd, b_minus=B2)
+    assert torch.all((c.double().cpu() - want).abs() <= bound)
+    rc = K.lib().mr_gemm_f32(K.GEMM_LAYOUT[layout], M, N, Kd, A.data_ptr(), A.stride(0), B.data_ptr(), B2.data_ptr(),
+                             B.stride(0), c.data_ptr(), N, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    assert torch.all((c.double().cpu() - want).abs() <= bound)
+
+
+# Values outside the three-plane split's range: infinities, NaNs, magnitudes at
+# the top of float32 and far below its normal range come out as float32 has them.
+@pytest.mark.parametrize("layout", ["nt", "tn"])
+@pytest.mark.parametrize("kind", ["inf", "nan", "huge", "tiny"])
+def test_gemm_f32_range(layout, kind):
+    M, N, Kd = 140, 136, 608
+    print("case gemm f32 range", layout, kind, flush=True, file=sys.stderr)
+    g = torch.Generator().manual_seed(5)
+    a, b = torch.randn(M, Kd, generator=g), torch.randn(N, Kd, generator=g)
+    if kind == "tiny":
+        a *= 1e-37
+    else:
+        a[133, 40] = {"inf": float("inf"), "nan": float("nan"), "huge": 3.4e38}[kind]
+        b[3, 40], b[4, 40], b[5, 40] = 0.0, -1.5, 0.5
+    want = a.double() @ b.double().T
+    A = (a if layout != "tn" else a.T.contiguous()).to(dev())
+    B = (b if layout == "nt" else b.T.contiguous()).to(dev())
+    c = torch.empty(M, N, device=dev())
+    K.gemm_f32(layout, A, B, c, M=M, N=N, K=Kd)
+    got = c.double().cpu()
+    ref = want.float().double()
+    assert torch.equal(got.isnan(), ref.isnan())
+    assert torch.equal(got.isinf(), ref.isinf()) and torch.equal(got[got.isinf()], ref[ref.isinf()])
+    fine = ref.isfinite()
+    # (2^-149 per term where products fall among the denormals)
+    bound = (Kd + 4) * 2.0**-23 * (a.double().abs() @ b.double().abs().T) + Kd * 2.0**-149
+    assert torch.all((got - want).abs()[fine] <= bound[fine])
