@@ -107,6 +107,15 @@ __device__ __forceinline__ void tile_coords(int lt, int grid_m, int grid_n, int&
   bn = (lt % per_group) / gm;
 }
 
+// Block i of n, renumbered so that each XCD (blocks are dealt to the eight
+// round-robin) works through one contiguous run, whatever n. (Only multiples of
+// eight renumbered before: 16384 x 960 x 576 41 us on small tiles, 22 now;
+// 1024 x 3584 x 37888 298 -> 245.)
+__device__ __forceinline__ int xcd_order(int i, int n) {
+  const int x = i & 7;
+  return x * (n >> 3) + min(x, n & 7) + (i >> 3);
+}
+
 typedef __attribute__((address_space(3))) void lds_void_t;
 
 // The wave's index in its block as a scalar, so that what derives from it
@@ -532,6 +541,23 @@ __device__ __forceinline__ void store_tile(const GemmParams& p, f32x16 (&acc)[TM
   }
 }
 
+// A k-split block's raw partial tile, for the reduce kernel: 32 x 32 blocks row
+// by row, each as the accumulators hold it (register group gi of the 64 lanes
+// contiguous), so that every store is a whole 1 KB. bi, bj: the wave's first
+// block.
+template <int BM, int BN, int TM, int TN>
+__device__ __forceinline__ void store_partial(float* out, const f32x16 (&acc)[TM][TN], int bi, int bj, int lane) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int gi = 0; gi < 4; ++gi)
+        *reinterpret_cast<f32x4*>(out + (((bi + i) * (BN / 32) + bj + j) * 4 + gi) * 256 + lane * 4) =
+            f32x4{acc[i][j][4 * gi], acc[i][j][4 * gi + 1], acc[i][j][4 * gi + 2], acc[i][j][4 * gi + 3]};
+}
+
 template <int BM, int BN, bool A_KMAJOR, bool B_KMAJOR, int EPI, bool OUT_BF16>
 __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmParams p) {
   constexpr int WM = BM / kWaveRows, WN = BN / (kWaves / kWaveRows);
@@ -552,15 +578,14 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmParams p) {
   __shared__ __attribute__((aligned(1024))) uint8_t Bs0[BN * ROW_BYTES];
   __shared__ __attribute__((aligned(1024))) uint8_t Bs1[BN * ROW_BYTES];
 
-  // XCD-aware renumbering (each XCD gets a contiguous run of the launch's
-  // tiles), then the grouped order along M. Split launches take the splits
-  // of one tile as consecutive blocks.
+  // XCD-aware renumbering, then the grouped order along M. Split launches take
+  // the splits of one tile as consecutive blocks.
   int bid = blockIdx.x, split = 0;
   if (p.ksplit > 1) {
     split = bid % p.ksplit;
     bid /= p.ksplit;
-  } else if ((p.n_tiles & 7) == 0) {
-    bid = (bid & 7) * (p.n_tiles >> 3) + (bid >> 3);
+  } else {
+    bid = xcd_order(bid, p.n_tiles);
   }
   int bm, bn;
   if (p.sub) {
@@ -722,25 +747,8 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmParams p) {
   }
 
   // ---- epilogue ----
-  const int lrow = (lane >> 5) * 4;
-  const int lcol = lane & 31;
-  if (p.ksplit > 1) {  // raw partial tile; the reduce kernel applies the epilogue
-    float* out = p.ws + (static_cast<int64_t>(bid) * p.ksplit + split) * (BM * BN);
-    auto tile = [&](auto ij) {
-      constexpr int i = decltype(ij)::value / TN, j = decltype(ij)::value % TN;
-      if constexpr (SWAP) {
-#pragma unroll
-        for (int gi = 0; gi < 4; ++gi)
-          *reinterpret_cast<float4*>(out + (wm * WM + i * 32 + lcol) * BN + wn * WN + j * 32 + gi * 8 + lrow) =
-              make_float4(acc[i][j][4 * gi], acc[i][j][4 * gi + 1], acc[i][j][4 * gi + 2], acc[i][j][4 * gi + 3]);
-      } else {
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          out[(wm * WM + i * 32 + (r >> 2) * 8 + lrow + (r & 3)) * BN + wn * WN + j * 32 + lcol] =
-              acc[i][j][r];
-      }
-    };
-    StaticFor<0, TM * TN>::run(tile);
+  if (p.ksplit > 1) {
+    store_partial<BM, BN>(p.ws + (static_cast<int64_t>(bid) * p.ksplit + split) * (BM * BN), acc, wm * TM, wn * TN, lane);
     return;
   }
   {
@@ -789,8 +797,8 @@ __global__ __launch_bounds__(64 * kWaves4) __attribute__((amdgpu_waves_per_eu(1,
   if (p.ksplit > 1) {
     split = bid % p.ksplit;
     bid /= p.ksplit;
-  } else if ((p.n_tiles & 7) == 0) {
-    bid = (bid & 7) * (p.n_tiles >> 3) + (bid >> 3);
+  } else {
+    bid = xcd_order(bid, p.n_tiles);
   }
   int bm, bn;
   tile_coords(p.tile0 + bid, p.grid_m, p.grid_n, bm, bn);
@@ -978,91 +986,310 @@ __global__ __launch_bounds__(64 * kWaves4) __attribute__((amdgpu_waves_per_eu(1,
   // the repeated last loads land, every wave is past its reads: LDS is free
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
-  if (p.ksplit > 1) {  // raw partial tile; the reduce kernel applies the epilogue
-    typedef float f32x4 __attribute__((ext_vector_type(4)));
-    float* out = p.ws + (static_cast<int64_t>(bid) * p.ksplit + split) * (BM * BN);
-    const int lrow = (lane >> 5) * 4, lcol = lane & 31;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int gi = 0; gi < 4; ++gi)
-          *reinterpret_cast<f32x4*>(out + (wm * WM + i * 32 + lcol) * BN + wn * WN + j * 32 + gi * 8 + lrow) =
-              f32x4{acc[i][j][4 * gi], acc[i][j][4 * gi + 1], acc[i][j][4 * gi + 2], acc[i][j][4 * gi + 3]};
+  if (p.ksplit > 1) {
+    store_partial<BM, BN>(p.ws + (static_cast<int64_t>(bid) * p.ksplit + split) * (BM * BN), acc, wm * TM, wn * TN, lane);
     return;
   }
   uint8_t* region = wave == 0 ? As0 : wave == 1 ? As1 : wave == 2 ? As2 : Bs0;
   store_tile<WM, WN, STAGE, EPI, OUT_BF16>(p, acc, m0, n0, wm, wn, lane, region);
 }
 
-// Sums the k-split partial tiles of a launch in split order and applies the
-// epilogue the whole-K kernel would have: one thread per 4 columns of a tile
-// row (for SwiGLU, per 4 act columns: gate and up sit 32 columns apart).
-template <int BM, int BN, int EPI, bool OUT_BF16>
-__global__ __launch_bounds__(256) void gemm_reduce(GemmParams p) {
-  constexpr int CW = EPI == EPI_SWIGLU ? BN / 2 : BN;  // output columns per tile
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  const int64_t per_tile = static_cast<int64_t>(BM) * (CW / 4);
-  if (idx >= per_tile * p.n_tiles) return;
-  const int t = static_cast<int>(idx / per_tile);
-  const int rem = static_cast<int>(idx % per_tile);
-  const int r = rem / (CW / 4), c4 = (rem % (CW / 4)) * 4;
+// ---- 4-wave kernel for 128 x 128 tiles on grids of at most one block per CU --
+//
+// Where a launch has no more tiles than CUs (the small models' products, cut
+// along K or not), nothing but a block's own loads can hide the memory latency:
+// the double-buffered kernel spends about 0.7 us on each 64-k tile of 0.2 us
+// of MFMAs. Here a block has the CU's LDS to itself: four stages of 32 KB, so
+// that three k-tiles are in flight while one is multiplied. One wave per SIMD
+// owns 64 x 64. As in the 256 x 256 kernel, the k-tile's barrier stands ahead
+// of its last k16 step: every wave has then read the stage in full, so the
+// loads of k-tile u + 4 go into it at once, half behind that step's MFMAs and
+// half behind the next k-tile's first, and the next k-tile's first operands
+// are read while the last step multiplies. What bounds it then is LDS: 64 KB
+// of operand reads and 32 KB of loads a k-tile, 0.33 us with few CUs at work
+// (0.2 us of MFMAs) and 0.42 with all 256 (measured, K = 4096).
+// Measured against the two-per-CU form: 576 x 576 x 4096 (25 tiles) 45 us, 26
+// here whole and 16 cut in 5; 4096 x 576 x 3072 34 -> 22; the residual products
+// 4096 x 576 x 1536 22 -> 16 and, on large tiles, 36; 2048 x 2048 x 2048 28 -> 20.
+template <bool A_KMAJOR, bool B_KMAJOR, int EPI, bool OUT_BF16>
+__global__ __launch_bounds__(64 * kWaves4) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_deep_kernel(GemmParams p) {
+  constexpr int BM = 128, BN = 128, WM = 64, WN = 64, TM = 2, TN = 2;
+  constexpr int STAGE = BM * ROW_BYTES;
+  __shared__ __attribute__((aligned(1024))) uint8_t As0[STAGE];
+  __shared__ __attribute__((aligned(1024))) uint8_t As1[STAGE];
+  __shared__ __attribute__((aligned(1024))) uint8_t As2[STAGE];
+  __shared__ __attribute__((aligned(1024))) uint8_t As3[STAGE];
+  __shared__ __attribute__((aligned(1024))) uint8_t Bs0[STAGE];
+  __shared__ __attribute__((aligned(1024))) uint8_t Bs1[STAGE];
+  __shared__ __attribute__((aligned(1024))) uint8_t Bs2[STAGE];
+  __shared__ __attribute__((aligned(1024))) uint8_t Bs3[STAGE];
+
+  // The first p.tile0 blocks take a whole tile each, the rest the (split, tile)
+  // pairs of the tail, tiles fastest: each XCD a contiguous run of either, so
+  // that its blocks share operand panels.
+  const bool cut = static_cast<int>(blockIdx.x) >= p.tile0;
+  const int blocks = cut ? p.n_tiles * p.ksplit : p.tile0;
+  int bid = static_cast<int>(blockIdx.x) - (cut ? p.tile0 : 0);
+  bid = xcd_order(bid, blocks);
+  const int split = cut ? bid / p.n_tiles : 0;
+  bid -= split * p.n_tiles;
   int bm, bn;
-  tile_coords(p.tile0 + t, p.grid_m, p.grid_n, bm, bn);
-  const int row = bm * BM + r;
-  if (row >= p.M) return;
-  const float* part = p.ws + static_cast<int64_t>(t) * p.ksplit * (BM * BN) + r * BN;
-  auto sum4 = [&](int c) {  // columns c .. c + 3 of the tile, splits in order
-    float4 a = *reinterpret_cast<const float4*>(part + c);
-    for (int sp = 1; sp < p.ksplit; ++sp) {
-      const float4 b = *reinterpret_cast<const float4*>(part + static_cast<int64_t>(sp) * (BM * BN) + c);
-      a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
-    }
-    return a;
+  tile_coords((cut ? p.tile0 : 0) + bid, p.grid_m, p.grid_n, bm, bn);
+  const int m0 = bm * BM, n0 = bn * BN;
+  const int lane = threadIdx.x & 63;
+  const int wave = wave_id();
+  const int wm = wave >> 1, wn = wave & 1;
+
+  std::conditional_t<A_KMAJOR, KMajorDirect<BM>, MNMajorDirect<BM>> ld_a;
+  std::conditional_t<B_KMAJOR, KMajorDirect<BN>, MNMajorDirect<BN>> ld_b;
+  ld_a.init(p.lda, m0, p.M);
+  ld_b.init(p.ldb, n0, p.N);
+  const int kt0 = split * p.kt_per;
+  const int KT = cut ? min(p.K / BK - kt0, p.kt_per) : p.K / BK;  // this block's k-tiles: kt0 .. kt0 + KT - 1
+  // The k-tile being loaded: its operands' first elements. Offsets from them
+  // are clamped inside the operands by the loaders, and the k-tiles stop at the
+  // last (loads past it repeat it into a stage nobody reads again).
+  const int64_t step_a = A_KMAJOR ? BK : BK * p.lda, step_b = B_KMAJOR ? BK : BK * p.ldb;
+  const uint16_t* at_a = p.A + (A_KMAJOR ? m0 * p.lda : m0) + kt0 * step_a;
+  const uint16_t* at_b = p.B + (B_KMAJOR ? n0 * p.ldb : n0) + kt0 * step_b;
+  auto advance = [&](int u) __attribute__((always_inline)) {  // to k-tile u
+    at_a += u < KT ? step_a : 0;
+    at_b += u < KT ? step_b : 0;
   };
-  if constexpr (EPI == EPI_SWIGLU) {
-    const int gc = (c4 / 32) * 64 + c4 % 32;  // tile column of the gate
-    const float4 g4 = sum4(gc), u4 = sum4(gc + 32);
-    const float gs[4] = {g4.x, g4.y, g4.z, g4.w}, us[4] = {u4.x, u4.y, u4.z, u4.w};
-    uint16_t* act = static_cast<uint16_t*>(p.C);
+
+  f32x16 acc[TM][TN];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int col = (bn * BN) / 2 + c4 + k;
-      const int gcol = bn * BN + gc + k;
-      if (col >= p.n_out) continue;
-      act[static_cast<int64_t>(row) * p.ldc + col] = f32_to_bf16(silu(gs[k]) * us[k]);
-      if (p.gu) {
-        p.gu[static_cast<int64_t>(row) * p.ldgu + gcol] = f32_to_bf16(gs[k]);
-        p.gu[static_cast<int64_t>(row) * p.ldgu + gcol + 32] = f32_to_bf16(us[k]);
-      }
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x16{};
+
+  // fragment addresses, as in the 8-wave kernel
+  constexpr int NA = A_KMAJOR ? BK / 16 : TM, NB = B_KMAJOR ? BK / 16 : TN;
+  uint32_t a_reg[NA], b_reg[NB];
+  {
+    const int h = lane >> 5, l32 = lane & 31;
+#pragma unroll
+    for (int x = 0; x < NA; ++x) {
+      if constexpr (A_KMAJOR)
+        a_reg[x] = (wm * WM + l32) * ROW_BYTES + (((2 * x + h) ^ swz_bits(l32)) << 4);
+      else
+        a_reg[x] = MNMajorDirect<BM>::frag_off(wm * WM + x * 32, lane);
+      asm volatile("" : "+v"(a_reg[x]));
     }
-  } else {
-    const float4 v4 = sum4(c4);
-    const float vs[4] = {v4.x, v4.y, v4.z, v4.w};
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int col = bn * BN + c4 + k;
-      if (col >= p.N) continue;
-      if constexpr (EPI == EPI_SWIGLU_BWD) {
-        const int gcol = (col >> 5) * 64 + (col & 31);
-        const int64_t o = static_cast<int64_t>(row) * p.ldgu + gcol;
-        const float g = bf16_to_f32(p.gu[o]), u = bf16_to_f32(p.gu[o + 32]);
-        const float sg = sigmoid(g);
-        const float dsilu = sg * (1.0f + g * (1.0f - sg));
-        uint16_t* dgu = static_cast<uint16_t*>(p.C);
-        const int64_t od = static_cast<int64_t>(row) * p.ldc + gcol;
-        dgu[od] = f32_to_bf16(vs[k] * u * dsilu);
-        dgu[od + 32] = f32_to_bf16(vs[k] * g * sg);
-      } else {
-        float x = vs[k] + (p.bias ? p.bias[col] : 0.0f);
-        if constexpr (EPI == EPI_RESID) x = p.resid[static_cast<int64_t>(row) * p.ldr + col] + x;
-        const int64_t o = static_cast<int64_t>(row) * p.ldc + col;
-        if constexpr (OUT_BF16) static_cast<uint16_t*>(p.C)[o] = f32_to_bf16(x);
-        else static_cast<float*>(p.C)[o] = x;
-      }
+    for (int x = 0; x < NB; ++x) {
+      if constexpr (B_KMAJOR)
+        b_reg[x] = (wn * WN + l32) * ROW_BYTES + (((2 * x + h) ^ swz_bits(l32)) << 4);
+      else
+        b_reg[x] = MNMajorDirect<BN>::frag_off(wn * WN + x * 32, lane);
+      asm volatile("" : "+v"(b_reg[x]));
     }
   }
+  typedef const __attribute__((address_space(3))) uint8_t* lds_ptr;
+  bf16x8 af[2][TM], bfr[2][TN];
+  auto rd_tr = [](lds_ptr l, uint32_t reg, int kk) __attribute__((always_inline)) {
+    constexpr uint32_t R = MNMajorDirect<128>::ROWB;
+    const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t*)(l + reg + kk * 16 * R));
+    const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t*)(l + reg + kk * 16 * R + 4 * R));
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+  auto rd = [&](lds_ptr la, lds_ptr lb, int kk, int slot) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      if constexpr (A_KMAJOR) af[slot][i] = *(const lds_bf16x8_t*)(la + a_reg[kk] + i * 32 * ROW_BYTES);
+      else af[slot][i] = rd_tr(la, a_reg[i], kk);
+    }
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      if constexpr (B_KMAJOR) bfr[slot][j] = *(const lds_bf16x8_t*)(lb + b_reg[kk] + j * 32 * ROW_BYTES);
+      else bfr[slot][j] = rd_tr(lb, b_reg[j], kk);
+    }
+  };
+  auto mm = [&](int slot) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[slot][j], af[slot][i], acc[i][j], 0, 0, 0);
+  };
+  // The order of a k16 step: the next step's fragment reads and the loads
+  // between its 4 MFMAs.
+  constexpr int NR = (A_KMAJOR ? TM : 2 * TM) + (B_KMAJOR ? TN : 2 * TN);
+  auto order = [](bool loads) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (q < 2) __builtin_amdgcn_sched_group_barrier(0x100, NR / 2, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      if (loads) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto issue = [&](uint8_t* a, uint8_t* b, int i0, int i1) __attribute__((always_inline)) {
+    const rsrc_t r_a = make_rsrc(at_a, 0x7fffffff), r_b = make_rsrc(at_b, 0x7fffffff);
+#pragma unroll
+    for (int i = i0; i < i1; ++i) {
+      ld_a.issue_one(r_a, i, a);
+      ld_b.issue_one(r_b, i, b);
+    }
+  };
+  const int phase = (4 - KT % 4) % 4;  // the stage k-tile 0 takes
+  {
+    auto pro = [&](uint8_t* a0, uint8_t* b0, uint8_t* a1, uint8_t* b1, uint8_t* a2, uint8_t* b2, uint8_t* a3,
+                   uint8_t* b3) __attribute__((always_inline)) {
+      issue(a0, b0, 0, 4);
+      advance(1);
+      issue(a1, b1, 0, 4);
+      advance(2);
+      issue(a2, b2, 0, 4);
+      advance(3);
+      issue(a3, b3, 0, 2);
+      asm volatile("s_waitcnt vmcnt(20)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      rd((lds_ptr)a0, (lds_ptr)b0, 0, 0);
+    };
+    switch (phase) {
+      case 0: pro(As0, Bs0, As1, Bs1, As2, Bs2, As3, Bs3); break;
+      case 1: pro(As1, Bs1, As2, Bs2, As3, Bs3, As0, Bs0); break;
+      case 2: pro(As2, Bs2, As3, Bs3, As0, Bs0, As1, Bs1); break;
+      default: pro(As3, Bs3, As0, Bs0, As1, Bs1, As2, Bs2); break;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // k-tile u, in stage S
+  auto tile = [&](int u, auto sc) __attribute__((always_inline)) {
+    constexpr int S = decltype(sc)::value;
+    uint8_t* la_ = S == 0 ? As0 : S == 1 ? As1 : S == 2 ? As2 : As3;
+    uint8_t* lb_ = S == 0 ? Bs0 : S == 1 ? Bs1 : S == 2 ? Bs2 : Bs3;
+    uint8_t* na_ = S == 0 ? As1 : S == 1 ? As2 : S == 2 ? As3 : As0;  // k-tile u + 1
+    uint8_t* nb_ = S == 0 ? Bs1 : S == 1 ? Bs2 : S == 2 ? Bs3 : Bs0;
+    uint8_t* pa_ = S == 0 ? As3 : S == 1 ? As0 : S == 2 ? As1 : As2;  // k-tile u + 3
+    uint8_t* pb_ = S == 0 ? Bs3 : S == 1 ? Bs0 : S == 2 ? Bs1 : Bs2;
+    const lds_ptr la = (lds_ptr)la_, lb = (lds_ptr)lb_;
+    rd(la, lb, 1, 1);
+    issue(pa_, pb_, 2, 4);
+    mm(0);
+    order(true);
+    rd(la, lb, 2, 0);
+    mm(1);
+    order(false);
+    rd(la, lb, 3, 1);
+    advance(u + 4);
+    mm(0);
+    order(false);
+    // Every read of this stage done, k-tile u + 1 landed (the 16 loads of
+    // k-tiles u + 2 and u + 3 may be in flight): a plain barrier, no fence.
+    asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    rd((lds_ptr)na_, (lds_ptr)nb_, 0, 0);
+    issue(la_, lb_, 0, 2);
+    mm(1);
+    order(true);
+  };
+  int u = 0;
+  if (phase <= 0) tile(u++, std::integral_constant<int, 0>{});
+  if (phase <= 1) tile(u++, std::integral_constant<int, 1>{});
+  if (phase <= 2) tile(u++, std::integral_constant<int, 2>{});
+  tile(u++, std::integral_constant<int, 3>{});
+  for (; u < KT; u += 4) {
+    tile(u, std::integral_constant<int, 0>{});
+    tile(u + 1, std::integral_constant<int, 1>{});
+    tile(u + 2, std::integral_constant<int, 2>{});
+    tile(u + 3, std::integral_constant<int, 3>{});
+  }
+  // the repeated last loads land, every wave is past its reads: LDS is free
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  if (cut && p.ksplit > 1) {
+    store_partial<BM, BN>(p.ws + (static_cast<int64_t>(bid) * p.ksplit + split) * (BM * BN), acc, wm * TM, wn * TN, lane);
+    return;
+  }
+  uint8_t* region = wave == 0 ? As0 : wave == 1 ? As1 : wave == 2 ? As2 : As3;
+  store_tile<WM, WN, STAGE, EPI, OUT_BF16>(p, acc, m0, n0, wm, wn, lane, region);
+}
+
+// Sums the k-split partial tiles of a launch in split order and applies the
+// epilogue the whole-K kernel would have. A block of 256 threads takes a
+// 32 x 32 block of a tile (for SwiGLU a pair: gate and up sit 32 columns
+// apart), a thread 4 columns of a row: the partials and the outputs both move
+// in whole 128-byte lines. (Against row-major partials and element-wise output:
+// the 3B split-precision products' reduces 33 -> 24 and 31 -> 25 us.)
+template <int BM, int BN, int EPI, bool OUT_BF16>
+__global__ __launch_bounds__(256) void gemm_reduce(GemmParams p) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  constexpr int NB = EPI == EPI_SWIGLU ? BN / 64 : BN / 32;  // blocks (or pairs) across a tile
+  constexpr int PER_TILE = (BM / 32) * NB;
+  const int t = static_cast<int>(blockIdx.x) / PER_TILE, rem = static_cast<int>(blockIdx.x) % PER_TILE;
+  const int bi = rem / NB, bj = rem % NB;
+  int bm, bn;
+  tile_coords(p.tile0 + t, p.grid_m, p.grid_n, bm, bn);
+  const int r = threadIdx.x >> 3, c = threadIdx.x & 7;  // row and 4-column piece of the block
+  const int row = bm * BM + bi * 32 + r;
+  if (row >= p.M) return;
+  auto sum4 = [&](int b) __attribute__((always_inline)) {  // piece of block column b, splits in order
+    const float* part = p.ws + static_cast<int64_t>(t) * p.ksplit * (BM * BN) +
+                        ((bi * (BN / 32) + b) * 4 + (c >> 1)) * 256 + ((c & 1) * 32 + r) * 4;
+    f32x4 a = *reinterpret_cast<const f32x4*>(part);
+#pragma unroll 4
+    for (int sp = 1; sp < p.ksplit; ++sp) a += *reinterpret_cast<const f32x4*>(part + static_cast<int64_t>(sp) * (BM * BN));
+    return a;
+  };
+  auto pack4 = [](f32x4 v) { return make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])); };
+  if constexpr (EPI == EPI_SWIGLU) {
+    const int col = (bn * BN) / 2 + bj * 32 + c * 4;  // act column; N and n_out are multiples of 32
+    if (col >= p.n_out) return;
+    const f32x4 g = sum4(2 * bj), u = sum4(2 * bj + 1);
+    f32x4 a;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) a[k] = silu(g[k]) * u[k];
+    *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.C) + static_cast<int64_t>(row) * p.ldc + col) = pack4(a);
+    if (p.gu) {
+      uint16_t* o = p.gu + static_cast<int64_t>(row) * p.ldgu + bn * BN + bj * 64 + c * 4;
+      *reinterpret_cast<uint2*>(o) = pack4(g);
+      *reinterpret_cast<uint2*>(o + 32) = pack4(u);
+    }
+  } else {
+    const int col = bn * BN + bj * 32 + c * 4;
+    if (col >= p.N) return;  // N is a multiple of 8: the piece lies wholly inside or past the edge
+    f32x4 x = sum4(bj);
+    if constexpr (EPI == EPI_SWIGLU_BWD) {
+      const int gcol = (col >> 5) * 64 + (col & 31);
+      const uint16_t* gu = p.gu + static_cast<int64_t>(row) * p.ldgu + gcol;
+      const uint2 gv = *reinterpret_cast<const uint2*>(gu), uv = *reinterpret_cast<const uint2*>(gu + 32);
+      f32x4 dg, du;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t gw = k < 2 ? gv.x : gv.y, uw = k < 2 ? uv.x : uv.y;
+        const float g = __uint_as_float((k & 1) ? (gw & 0xffff0000u) : (gw << 16));
+        const float u = __uint_as_float((k & 1) ? (uw & 0xffff0000u) : (uw << 16));
+        const float sg = sigmoid(g);
+        const float dsilu = sg * (1.0f + g * (1.0f - sg));
+        dg[k] = x[k] * u * dsilu;
+        du[k] = x[k] * g * sg;
+      }
+      uint16_t* o = static_cast<uint16_t*>(p.C) + static_cast<int64_t>(row) * p.ldc + gcol;
+      *reinterpret_cast<uint2*>(o) = pack4(dg);
+      *reinterpret_cast<uint2*>(o + 32) = pack4(du);
+    } else {
+      if (p.bias) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) x[k] += p.bias[col + k];
+      }
+      const int64_t o = static_cast<int64_t>(row) * p.ldc + col;
+      if constexpr (EPI == EPI_RESID)
+        x = *reinterpret_cast<const f32x4*>(p.resid + static_cast<int64_t>(row) * p.ldr + col) + x;
+      if constexpr (OUT_BF16) *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.C) + o) = pack4(x);
+      else *reinterpret_cast<f32x4*>(static_cast<float*>(p.C) + o) = x;
+    }
+  }
+}
+
+template <int BM, int BN, int EPI, bool OUT_BF16>
+void launch_reduce(const GemmParams& p, hipStream_t s) {
+  constexpr int PER_TILE = (BM / 32) * (EPI == EPI_SWIGLU ? BN / 64 : BN / 32);
+  hipLaunchKernelGGL((gemm_reduce<BM, BN, EPI, OUT_BF16>), dim3(static_cast<unsigned>(p.n_tiles) * PER_TILE), dim3(256),
+                     0, s, p);
 }
 
 // The k-split tails' partial tiles live in a workspace the caller passes in
@@ -1091,16 +1318,106 @@ int split_plan(int64_t tiles, int KT, int64_t ws_bytes) {
   return split;
 }
 
-// Bytes of partials the plan uses for an M x N x K product (0: no split).
+// How a product runs is whichever of three plans the times below expect to
+// take least. The constants are microseconds, fitted to 237 products (the
+// eleven of a block over geometries of hidden 512 .. 3584 and 256 .. 16384
+// tokens, and the vocabulary heads), each run by every plan: median error 4-6 %,
+// and the plan chosen is on average 1.3 % slower than the best of them. The
+// start and epilogue of a round of tiles depend on the kind of output.
+enum Output { OUT_B16, OUT_F32, OUT_RESID, OUT_SWIGLU, OUT_SWIGLU_BWD, OUTPUTS };
+
+// 128 x 128 tiles on the deep kernel, one block per CU: rounds of 256 tiles, the
+// tail past them cut along K into `split` blocks a tile, whose partials take a
+// round trip and a second kernel. A k-tile takes longer the more CUs work.
+double deep_time(int64_t tiles, int KT, int split, Output o) {
+  constexpr double start[OUTPUTS] = {2.4, 2.9, 3.9, 3.8, 5.0};
+  const int64_t tail = tiles % 256, blocks = tail * split;
+  double t = 2.6 + static_cast<double>(tiles / 256) * (start[o] + 0.467 * KT);
+  if (tail) t += start[o] + (KT + split - 1) / split * (0.26 + 0.207 * static_cast<double>(blocks) / 256.0);
+  if (split > 1) t += 2.2 + 0.027 * static_cast<double>(blocks);
+  return t;
+}
+
+// The double-buffered 128 x 128 tiles, two blocks per CU: rounds of 512.
+double small_time(int64_t tiles, int KT, Output o) {
+  constexpr double start[OUTPUTS] = {1.1, 2.8, 3.2, 2.5, 5.9};
+  const int64_t r = tiles % 512;
+  double t = 1.5 + static_cast<double>(tiles / 512) * (start[o] + 1.024 * KT);
+  if (r) t += start[o] + KT * (r <= 256 ? 0.601 : 0.749 + 0.275 * static_cast<double>(r - 256) / 256.0);
+  return t;
+}
+
+// 256 x 256 tiles, one per CU: rounds of 256, the tail in `split` blocks a tile
+// or, up to half a round of plain stores, as quarter tiles (see launch).
+double big_time(int64_t tiles, int KT, int split, Output o) {
+  constexpr double start[OUTPUTS] = {8.2, 9.4, 12.2, 10.3, 18.8};
+  const int64_t tail = tiles % 256, blocks = tail * split;
+  double t = static_cast<double>(tiles / 256) * (start[o] + 1.481 * KT);
+  if (tail && split == 1 && o <= OUT_F32 && tiles >= 256 && tail <= 128) {
+    t += start[o] + 0.66 * KT;
+  } else if (tail) {
+    const double busy = blocks < 256 ? static_cast<double>(blocks) / 256.0 : 1.0;
+    t += static_cast<double>((blocks + 255) / 256) * (start[o] + (KT + split - 1) / split * (0.84 + 0.641 * busy));
+  }
+  if (split > 1) t += 2.9 + 0.052 * static_cast<double>(blocks);
+  return t;
+}
+
+enum Kind { BIG, SMALL, DEEP };
+struct Plan {
+  Kind kind;
+  int split;  // DEEP: blocks per tail tile
+};
+
+// In longer runs than these the deep kernel's k-tile slows beyond the fit (to
+// 0.6 us: 1024 x 3584 x 37888 took 359 us against 262 on split large tiles,
+// 9728 x 896 x 16384, two whole rounds, 353 against 290).
+constexpr int kDeepMaxKt = 320, kDeepMaxKtRounds = 160;
+
+// The plan of an M x N x (64 KT) product with ws_bytes for partials.
+Plan plan_for(int64_t M, int64_t N, int KT, Output o, int64_t ws_bytes) {
+  const int64_t big = ((M + 255) / 256) * ((N + 255) / 256);
+  const int64_t small = ((M + 127) / 128) * ((N + 127) / 128);
+  Plan p{BIG, 1};
+  double best = big_time(big, KT, split_plan(big, KT, ws_bytes), o);
+  if (small_time(small, KT, o) < best) {
+    best = small_time(small, KT, o);
+    p.kind = SMALL;
+  }
+  const int64_t tail = small % 256;
+  for (int sp = 1; sp <= 16; ++sp) {
+    if (sp > 1 && (!tail || tail * sp > 256 || sp * 2 > KT || tail * sp * (128ll * 128 * 4) > ws_bytes)) break;
+    if ((KT + sp - 1) / sp > kDeepMaxKt || (small >= 256 && KT > kDeepMaxKtRounds)) continue;
+    const double t = deep_time(small, KT, sp, o);
+    if (t < best) {
+      best = t;
+      p = Plan{DEEP, sp};
+    }
+  }
+  return p;
+}
+
+// Bytes of partials the plan uses for an M x N x K product (0: no split),
+// whatever its output.
 int64_t split_bytes(int64_t M, int64_t N, int64_t K) {
   const int KT = static_cast<int>(K / BK);
-  if (KT < kSplitMinKt) return 0;  // short K: whole-K tiles of either size
-  const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
-  const int split = split_plan(tiles, KT, kSplitCapBytes);
-  if (split == 1) return 0;
-  const int kt_per = (KT + split - 1) / split;
-  const int ksplit = (KT + kt_per - 1) / kt_per;
-  return (tiles % 256) * ksplit * 256ll * 256 * 4;
+  int64_t bytes = 0;
+  for (int o = 0; o < OUTPUTS; ++o) {
+    const Plan p = plan_for(M, N, KT, static_cast<Output>(o), kSplitCapBytes);
+    int64_t b = 0;
+    if (p.kind == DEEP && p.split > 1) {
+      b = (((M + 127) / 128) * ((N + 127) / 128) % 256) * p.split * 128ll * 128 * 4;
+    } else if (p.kind == BIG) {
+      const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
+      const int split = split_plan(tiles, KT, kSplitCapBytes);
+      if (split > 1) {
+        const int kt_per = (KT + split - 1) / split;
+        b = (tiles % 256) * ((KT + kt_per - 1) / kt_per) * 256ll * 256 * 4;
+      }
+    }
+    bytes = b > bytes ? b : bytes;
+  }
+  return bytes;
 }
 
 // Large tiles go out in whole waves of 256 (one per CU). When K is long (at
@@ -1108,8 +1425,7 @@ int64_t split_bytes(int64_t M, int64_t N, int64_t K) {
 // round trip), a remainder that would leave CUs idle in a last, partial wave
 // (or a whole grid under one wave) is cut along K instead: ksplit blocks per
 // tile, chosen (up to 16) to minimise the remainder's time in tile units,
-// ceil(tail * ksplit / 256) / ksplit, within the workspace. (Small tiles run
-// two per CU and are not split: measured, the split did not pay for them.)
+// ceil(tail * ksplit / 256) / ksplit, within the workspace.
 // Whole 256 x 256 tiles tile0 .. tile0 + n - 1 of p, without a k split: the
 // 4-wave kernel (K of at least two k-tiles), else the 8-wave one.
 // MR_GEMM_8WAVE=1 in the environment keeps every launch on the 8-wave kernel
@@ -1189,38 +1505,53 @@ int launch(GemmParams p, hipStream_t s) {
   else
     hipLaunchKernelGGL((gemm_kernel<BM, BN, AK, BKM, EPI, OB>),
                        dim3(static_cast<unsigned>(tail * p.ksplit)), dim3(kThreads), 0, s, p);
-  constexpr int CW = EPI == EPI_SWIGLU ? BN / 2 : BN;
-  const int64_t threads = tail * BM * (CW / 4);
-  hipLaunchKernelGGL((gemm_reduce<BM, BN, EPI, OB>), dim3(static_cast<unsigned>((threads + 255) / 256)),
-                     dim3(256), 0, s, p);
+  launch_reduce<BM, BN, EPI, OB>(p, s);
   MR_LAUNCH_CHECK("mr_gemm");
   return MR_OK;
 }
 
-// Large tiles unless small ones finish sooner. A long K (at least
-// kSplitMinKt steps) always takes 256 x 256 tiles: a remainder wave, or a
-// grid under one wave, is cut along K (measured on the weight gradients of the
-// small models, M, N <= 3584 and K = 16384, and the short-sequence input
-// gradients: 1.1-3.6x faster than small tiles, which leave CUs idle when the
-// output is small). Otherwise the two sizes are compared in whole waves: 256
-// large tiles per wave, 512 small ones (two per CU), a wave of small tiles
-// taking kSmallWave of a large one's time at the same K (0.58 measured with
-// K = 3584; 0.45 for K <= 1024, where the prologue and epilogue of the two
-// co-resident small tiles overlap each other's k loops). Small tiles win for
-// K = 896 (the 0.5B block: its qkv projection 1.6x faster) and when large
-// ones leave a last wave mostly idle (the 3B qkv projection: 2.5 waves). The
-// residual epilogue (an fp32 read and write per output) stays on large tiles:
-// measured, the 0.5B o projection ran 1.2x slower on small ones.
+// Small tiles on the deep kernel: whole rounds of 256, then the tail cut along K.
+template <bool AK, bool BKM, int EPI, bool OB>
+int launch_deep(GemmParams p, int split, hipStream_t s) {
+  p.grid_m = (p.M + 127) / 128;
+  p.grid_n = (p.N + 127) / 128;
+  const int64_t tiles = static_cast<int64_t>(p.grid_m) * p.grid_n;
+  const int KT = p.K / BK;
+  p.n_tiles = static_cast<int>(tiles % 256);
+  p.tile0 = static_cast<int>(tiles) - p.n_tiles;
+  p.kt_per = (KT + split - 1) / split;
+  p.ksplit = (KT + p.kt_per - 1) / p.kt_per;  // no empty split
+  if (use_4wave(KT)) {
+    hipLaunchKernelGGL((gemm_deep_kernel<AK, BKM, EPI, OB>), dim3(static_cast<unsigned>(p.tile0 + p.n_tiles * p.ksplit)),
+                       dim3(64 * kWaves4), 0, s, p);
+  } else {  // the same tiles and splits on the 8-wave kernel
+    GemmParams q = p;
+    q.n_tiles = p.tile0;
+    q.tile0 = 0;
+    q.ksplit = 1;
+    q.kt_per = KT;
+    if (q.n_tiles)
+      hipLaunchKernelGGL((gemm_kernel<128, 128, AK, BKM, EPI, OB>), dim3(static_cast<unsigned>(q.n_tiles)), dim3(kThreads),
+                         0, s, q);
+    if (p.n_tiles)
+      hipLaunchKernelGGL((gemm_kernel<128, 128, AK, BKM, EPI, OB>), dim3(static_cast<unsigned>(p.n_tiles * p.ksplit)),
+                         dim3(kThreads), 0, s, p);
+  }
+  if (p.n_tiles && p.ksplit > 1) launch_reduce<128, 128, EPI, OB>(p, s);
+  MR_LAUNCH_CHECK("mr_gemm");
+  return MR_OK;
+}
+
 template <bool AK, bool BKM, int EPI, bool OB>
 int dispatch(GemmParams p, hipStream_t s) {
-  const int KT = p.K / BK;
-  if (KT >= kSplitMinKt) return launch<256, 256, AK, BKM, EPI, OB>(p, s);
-  const int64_t big = static_cast<int64_t>((p.M + 255) / 256) * ((p.N + 255) / 256);
-  const int64_t small = static_cast<int64_t>((p.M + 127) / 128) * ((p.N + 127) / 128);
-  const double wave_small = KT <= 16 ? 0.45 : 0.58;
-  const double t_big = static_cast<double>((big + 255) / 256);
-  const double t_small = static_cast<double>((small + 511) / 512) * wave_small;
-  if (EPI != EPI_RESID && t_small < 0.97 * t_big) return launch<128, 128, AK, BKM, EPI, OB>(p, s);
+  constexpr Output o = EPI == EPI_RESID        ? OUT_RESID
+                       : EPI == EPI_SWIGLU     ? OUT_SWIGLU
+                       : EPI == EPI_SWIGLU_BWD ? OUT_SWIGLU_BWD
+                       : OB                    ? OUT_B16
+                                               : OUT_F32;
+  const Plan plan = plan_for(p.M, p.N, p.K / BK, o, p.ws ? p.ws_bytes : 0);
+  if (plan.kind == DEEP) return launch_deep<AK, BKM, EPI, OB>(p, plan.split, s);
+  if (plan.kind == SMALL) return launch<128, 128, AK, BKM, EPI, OB>(p, s);
   return launch<256, 256, AK, BKM, EPI, OB>(p, s);
 }
 

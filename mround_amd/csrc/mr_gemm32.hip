@@ -239,7 +239,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_f32_kernel(Gemm32 p) {
   const int cut = blockIdx.x >= static_cast<unsigned>(p.full);
   const int blocks = cut ? p.tail * p.ksplit : p.full;
   int bid = static_cast<int>(blockIdx.x) - (cut ? p.full : 0);
-  if ((blocks & 7) == 0) bid = (bid & 7) * (blocks >> 3) + (bid >> 3);
+  bid = (bid & 7) * (blocks >> 3) + min(bid & 7, blocks & 7) + (bid >> 3);
   const int split = cut ? bid / p.tail : 0, tile = cut ? p.full + bid % p.tail : bid;
   const int m0 = (tile / p.grid_n) * TM, n0 = (tile % p.grid_n) * TN;
   const int k_lo = split * p.kt_per * TK;

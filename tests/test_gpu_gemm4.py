@@ -165,3 +165,75 @@ def test_4wave_k_split(layout, mnk):
     with _EightWave():
         K.gemm(layout, a, b, c8, M=M, N=N, K=Kd, workspace=ws)
     assert torch.equal(c, c8), "4-wave and 8-wave kernels differ"
+
+
+# The deep 128 x 128 kernel (four LDS stages) on small grids: every entry
+# position into the stage pattern and K shorter than it (KT = 1 .. 9), ragged
+# edges, a grid past one round whose tail is cut along K (258 tiles), and
+# k-split grids with every epilogue, against a float32 product within the
+# accumulation bound and bit for bit against the 8-wave kernel on the same
+# tiles and splits.
+@pytest.mark.parametrize("layout", ["nt", "nn", "tn"])
+@pytest.mark.parametrize("mnk", [(264, 328, 64 * kt) for kt in (1, 2, 3, 4, 5, 9)]
+                         + [(128, 128, 4096), (584, 568, 4160), (5504, 760, 1280)])
+@pytest.mark.parametrize("kind", ["f32", "bf16 bias", "resid"])
+def test_deep(layout, mnk, kind):
+    M, N, Kd = mnk
+    print("case deep", layout, mnk, kind, flush=True, file=sys.stderr)
+    a, b, a_ref, b_ref = _operands(layout, M, N, Kd, seed=180 + Kd // 64)
+    ref, bound = _gpu_ref(a_ref, b_ref)
+    bias = resid = None
+    if kind == "bf16 bias":
+        bias = torch.randn(N, generator=torch.Generator().manual_seed(182)).to(dev())
+        ref = ref + bias
+        bound = bound + ref.abs() * 2.0**-8
+    elif kind == "resid":
+        resid = torch.randn(M, N, generator=torch.Generator().manual_seed(183)).to(dev())
+        ref = resid + ref
+        bound = bound + ref.abs() * 2.0**-22
+    if Kd >= 4096:
+        assert K.gemm_workspace_bytes(M, N, Kd) > 0, "this shape is expected to split"
+    out = torch.bfloat16 if bias is not None else torch.float32
+    c = torch.full((M, N), 7.0, dtype=out, device=dev())
+    K.gemm(layout, a, b, c, M=M, N=N, K=Kd, bias=bias, resid=resid)
+    assert bool(torch.all((c.float() - ref).abs() <= bound))
+    c8 = torch.full((M, N), 5.0, dtype=out, device=dev())
+    with _EightWave():
+        K.gemm(layout, a, b, c8, M=M, N=N, K=Kd, bias=bias, resid=resid)
+    assert torch.equal(c, c8), "the deep and 8-wave kernels differ"
+
+
+@pytest.mark.parametrize("kd", [128, 2560])
+def test_deep_swiglu(kd):
+    M, n = 392, 352  # 4 x 6 and 4 x 3 tiles with ragged edges; K = 2560 is cut
+    print("case deep swiglu", kd, flush=True, file=sys.stderr)
+    x, wd = _rand(M, kd, seed=190).to(dev()), _rand(kd, n, seed=193).to(dev())
+    wgu = interleave_gate_up(_rand(n, kd, seed=191), _rand(n, kd, seed=192)).to(dev())
+    outs = []
+    for eight in (False, True):
+        act, gu, dgu = (torch.empty(M, w, dtype=torch.bfloat16, device=dev()) for w in (n, 2 * n, 2 * n))
+        if eight:
+            os.environ["MR_GEMM_8WAVE"] = "1"
+        try:
+            K.gemm_swiglu(x, wgu, act, gu)
+            K.gemm_swiglu_bwd(x, wd, gu, dgu)
+        finally:
+            os.environ.pop("MR_GEMM_8WAVE", None)
+        outs.append((act, gu, dgu))
+    assert all(torch.equal(p, q) for p, q in zip(*outs)), "the deep and 8-wave kernels differ"
+    act, gu, dgu = outs[0]
+    ref, bound = _gpu_ref(x, wgu.t().contiguous())
+    assert bool(torch.all((gu.float() - ref).abs() <= bound + ref.abs() * 2.0**-8))
+    g, u = (t.reshape(M, n) for t in gu.float().reshape(M, n // 32, 2, 32).unbind(2))
+    rg, ru = (t.reshape(M, n) for t in ref.reshape(M, n // 32, 2, 32).unbind(2))
+    bg, bu = (t.reshape(M, n) for t in bound.reshape(M, n // 32, 2, 32).unbind(2))
+    act_ref = torch.nn.functional.silu(rg) * ru
+    tol = 1.1 * bg * ru.abs() + bu * torch.nn.functional.silu(rg).abs() + act_ref.abs() * 2.0**-7 + 1e-6
+    assert bool(torch.all((act.float() - act_ref).abs() <= tol))
+    dact, bd = _gpu_ref(x, wd)
+    sg = torch.sigmoid(g)
+    want = torch.stack([(dact * u * sg * (1 + g * (1 - sg))).reshape(M, n // 32, 32),
+                        (dact * g * sg).reshape(M, n // 32, 32)], 2)
+    tol = torch.stack([(bd * u.abs() * 1.1).reshape(M, n // 32, 32), (bd * (g.abs() * sg)).reshape(M, n // 32, 32)], 2)
+    got = dgu.float().reshape(M, n // 32, 2, 32)
+    assert bool(torch.all((got - want).abs() <= tol + want.abs() * 2.0**-7 + 1e-6))
