@@ -112,3 +112,30 @@ def test_searched_block_tune_commits_bit_exact():
         assert np.array_equal(q.scale.cpu().numpy(), scale.reshape(q.scale.shape))
         assert np.array_equal(block.weights.linears[n].float().cpu().numpy(),
                               OQ.round_to_bf16(wq.astype(np.float32)))
+
+
+# Groups shared by 1 .. 32 lanes (the smallest matrices split the candidates
+# most), rows that do not fill a wave, and magnitudes at both ends of the range:
+# groups above 2^126 at 2 bits take the unfused residual.
+@pytest.mark.parametrize("bits", [2, 3])
+@pytest.mark.parametrize("shape", [(1, 32), (3, 128), (65, 256), (515, 128), (4100, 512)])
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("with_imp", [False, True])
+def test_search_splits_and_range(bits, shape, gs, with_imp):
+    rows, cols = shape
+    if cols % gs:
+        pytest.skip("the group does not divide the row")
+    print("case search split", bits, shape, gs, with_imp, flush=True, file=sys.stderr)
+    w = weight(rows, cols, seed=rows + bits, dtype=torch.float32)
+    if rows > 3:
+        w[0] *= 2.0**130
+        w[1] *= 1e-42 / 0.02
+        w[2] = 0
+        w[3] = w[3].clamp(-0.02, 0.02)  # ties at the anchor
+        w[rows - 1] *= 2.0**120
+    imp = (torch.rand(cols, generator=torch.Generator().manual_seed(gs)) * 10 + 0.1) if with_imp else None
+    scheme = QuantScheme(bits=bits, group_size=gs, symmetry=Symmetry.SYMMETRIC, scale_init=ScaleInit.SEARCHED)
+    got = search_scales(w.to(dev()), scheme, importance=None if imp is None else imp.to(dev())).cpu().numpy()
+    with np.errstate(all="ignore"):
+        want = OS.search_scales_f32(w.numpy(), bits, gs, importance=None if imp is None else imp.numpy())
+    assert np.array_equal(got, want)
