@@ -8,10 +8,10 @@
 // The threshold is found exactly by a two-pass radix select on the bit
 // pattern of |r| (non-negative floats order like their bit patterns, and the
 // sign bit is dropped): a histogram of the top 15 bits (30..16) built in LDS
-// per block, a one-block select of the bin holding the k-th largest, then a
-// histogram of the low 16 bits among the elements of that bin only (global
-// atomics, few elements), and a second select. Everything stays on the
-// device; no host synchronisation.
+// per block, a select of the bin holding the k-th largest, then a histogram of
+// the low 16 bits among the elements of that bin only (global atomics, few
+// elements), and a second select. Everything stays on the device; no host
+// synchronisation.
 //
 // One pass over the data in the common case. A guess comes first: the top
 // bits of the (2 ceil(k / 37) + 64)-th largest key in a sample of a 37th of
@@ -46,11 +46,11 @@ constexpr int kBlock = 256;
 constexpr int kBlocks = 1024;
 constexpr int kHiBits = 15, kLoBits = 16;
 constexpr int kHiBins = 1 << kHiBits, kLoBins = 1 << kLoBits;
-constexpr int kSelThreads = 1024;
 constexpr int kHistThreads = 1024;
 
 constexpr int kHistBlocks = 256;                             // the first pass's grid, at most
 constexpr int kCandWaves = kHistBlocks * (kHistThreads / 64);  // one candidate list per wave
+constexpr int kCopies = 8;
 constexpr int kCandCap = 128;                                 // candidates listed per wave
 struct Workspace {
   double partial[kBlocks];
@@ -65,9 +65,14 @@ struct Workspace {
   uint32_t cand_count[kCandWaves];
   uint32_t cand_idx[kCandWaves * kCandCap];
   float cand_r[kCandWaves * kCandCap];
+  // sums of 256 consecutive bins of the three histograms, for pick() (the
+  // data's few exponents share a few sums: block b adds to copy b % kCopies)
+  uint32_t coarse_s[kCopies][kHiBins / 256];
+  uint32_t coarse_hi[kCopies][kHiBins / 256];
+  uint32_t coarse_lo[kLoBins / 256];
 };
 constexpr size_t kScratchBytes = sizeof(Workspace);
-static_assert(kScratchBytes == 4778016, "the documented workspace size");
+static_assert(kScratchBytes == 4787232, "the documented workspace size");
 constexpr int64_t kMaxElements = 0xffffffffLL;  // histogram counts are 32-bit
 constexpr int kMaxDevices = 64;
 
@@ -94,12 +99,93 @@ __global__ __launch_bounds__(kBlock) void zero_hist(Workspace* ws, uint32_t k) {
     ws->hist_s[i] = 0;
   }
   if (i < kLoBins) ws->hist_lo[i] = 0;
+  if (i < kCopies * (kHiBins / 256)) (&ws->coarse_s[0][0])[i] = (&ws->coarse_hi[0][0])[i] = 0;
+  if (i < kLoBins / 256) ws->coarse_lo[i] = 0;
   if (i == 0) {
     ws->state[0] = 0;
     ws->state[1] = k;
     ws->state[3] = 0;
     ws->state[4] = 0xffffffffu;
   }
+}
+
+// Selects. Every block that needs one makes it itself, from the 256-bin sums and
+// then the 256 bins of the chosen sum: two reads of at most 1 KB in a wave
+// (1-2 us) in place of a kernel of one block that reads the whole histogram
+// (8.5-11 us and a launch, three times a loss; measured on the 0.5B batch of
+// 4 x 1000 tokens, the loss's kernels 71 us with them, 46 without).
+//
+// The bin holding the k-th largest: the largest b with count(bins > b) < k <=
+// count(bins >= b), and that count above it. wave_pick: among N * 64 bins, N a
+// lane, for a whole wave (each bin in COPIES arrays, one after the other).
+struct Picked {
+  uint32_t bin, above;
+};
+template <int N, int COPIES>
+__device__ __forceinline__ Picked wave_pick(const uint32_t* __restrict__ h, uint32_t k) {
+  const int lane = threadIdx.x & 63;
+  uint32_t c[N], mine = 0;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    c[j] = h[lane * N + j];
+#pragma unroll
+    for (int q = 1; q < COPIES; ++q) c[j] += h[q * (64 * N) + lane * N + j];
+    mine += c[j];
+  }
+  uint32_t suf = mine;  // this lane's bins and those above
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t v = __shfl_down(suf, off, 64);
+    if (lane + off < 64) suf += v;
+  }
+  uint32_t above = suf - mine;
+  Picked p{0, 0};
+  bool found = false;
+#pragma unroll
+  for (int j = N - 1; j >= 0; --j) {
+    if (above < k && k <= above + c[j]) {
+      p = Picked{static_cast<uint32_t>(lane * N + j), above};
+      found = true;
+    }
+    above += c[j];
+  }
+  const uint64_t m = __ballot(found);
+  const int src = m ? __builtin_ctzll(m) : 0;
+  return Picked{__shfl(p.bin, src, 64), __shfl(p.above, src, 64)};
+}
+
+// The pick over 64 N * 256 bins (coarse: their sums), for a whole block; `sh`
+// is two shared words.
+template <int N, int COPIES>
+__device__ __forceinline__ Picked pick(const uint32_t* __restrict__ coarse, const uint32_t* __restrict__ fine, uint32_t k,
+                                       uint32_t* sh) {
+  if (threadIdx.x < 64) {
+    const Picked c = wave_pick<N, COPIES>(coarse, k);
+    const Picked f = wave_pick<4, 1>(fine + c.bin * 256, k - c.above);
+    if (threadIdx.x == 0) {
+      sh[0] = c.bin * 256 + f.bin;
+      sh[1] = c.above + f.above;
+    }
+  }
+  __syncthreads();
+  return Picked{sh[0], sh[1]};
+}
+
+// A block's histogram of the top bits, in LDS, added to the global one and its
+// sums, the latter once per block (by way of `sums`; a wave's 64 consecutive
+// bins lie in one sum).
+__device__ __forceinline__ void flush_hist(const uint32_t* h, uint32_t* sums, uint32_t* __restrict__ hist,
+                                           uint32_t (*__restrict__ coarse)[kHiBins / 256]) {
+  for (int i = threadIdx.x; i < kHiBins; i += kHistThreads) {
+    const uint32_t c = h[i];
+    if (__ballot(c != 0) == 0) continue;
+    if (c) atomicAdd(&hist[i], c);
+    uint32_t t = c;
+    for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+    if ((threadIdx.x & 63) == 0) atomicAdd(&sums[i >> 8], t);
+  }
+  __syncthreads();
+  if (threadIdx.x < kHiBins / 256 && sums[threadIdx.x])
+    atomicAdd(&coarse[blockIdx.x % kCopies][threadIdx.x], sums[threadIdx.x]);
 }
 
 // The sample: every 37th run of 64 consecutive elements (whole 256-byte
@@ -118,7 +204,9 @@ __global__ __launch_bounds__(kHistThreads) void sample_hist(const float* __restr
                                                             const float* __restrict__ target, int64_t n,
                                                             Workspace* __restrict__ ws) {
   __shared__ uint32_t h[kHiBins];
+  __shared__ uint32_t sums[kHiBins / 256];
   for (int i = threadIdx.x; i < kHiBins; i += kHistThreads) h[i] = 0;
+  if (threadIdx.x < kHiBins / 256) sums[threadIdx.x] = 0;
   __syncthreads();
   const int64_t ns = sample_count(n);
   for (int64_t j = static_cast<int64_t>(blockIdx.x) * kHistThreads + threadIdx.x; j < ns;
@@ -127,22 +215,22 @@ __global__ __launch_bounds__(kHistThreads) void sample_hist(const float* __restr
     atomicAdd(&h[abs_key(pred[i] - target[i]) >> kLoBits], 1u);
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < kHiBins; i += kHistThreads)
-    if (h[i]) atomicAdd(&ws->hist_s[i], h[i]);
+  flush_hist(h, sums, ws->hist_s, ws->coarse_s);
 }
 
 // The candidate lists hold every element of the selected top-bits bin and above.
-__device__ __forceinline__ bool lists_cover(const Workspace* ws) {
-  return ws->state[3] == 0 && ws->state[4] <= (ws->state[0] << kLoBits);
+__device__ __forceinline__ bool lists_cover(const Workspace* ws, uint32_t digit) {
+  return ws->state[3] == 0 && ws->state[4] <= (digit << kLoBits);
 }
 
 // ... and the threshold is not a NaN (then |r| < t keeps nothing, which the
 // key order would not say), so the loss can be formed from the lists.
-__device__ __forceinline__ bool lists_serve_loss(const Workspace* ws) {
-  return lists_cover(ws) && ws->state[2] <= 0x7f800000u;
+__device__ __forceinline__ bool lists_serve_loss(const Workspace* ws, uint32_t digit, uint32_t key) {
+  return lists_cover(ws, digit) && key <= 0x7f800000u;
 }
 
-// Pass 1, fused: the histogram of key >> 16 over every element (per block in
+// Pass 1, fused: the guess from the sample (ks: its rank there, 0 for none),
+// the histogram of key >> 16 over every element (per block in
 // LDS, 128 KB, then the block's non-empty bins added to the global one), the
 // gradient of every element (2 r / denom, as if kept), r^2 summed over the
 // elements under the guess key, and each wave's candidates (index and r, in
@@ -152,12 +240,19 @@ __global__ __launch_bounds__(kHistThreads) void loss_first_pass(const float* __r
                                                                 const float* __restrict__ target,
                                                                 int64_t n, float grad_scale,
                                                                 float* __restrict__ grad,
-                                                                Workspace* __restrict__ ws) {
+                                                                Workspace* __restrict__ ws, uint32_t ks) {
   __shared__ uint32_t h[kHiBins];
   __shared__ double smem[kHistThreads / 64];
+  __shared__ uint32_t sh[2];
+  __shared__ uint32_t sums[kHiBins / 256];
   for (int i = threadIdx.x; i < kHiBins; i += kHistThreads) h[i] = 0;
+  if (threadIdx.x < kHiBins / 256) sums[threadIdx.x] = 0;
+  uint32_t gkey = 0xffffffffu;
+  if (ks) {
+    gkey = pick<2, kCopies>(&ws->coarse_s[0][0], ws->hist_s, ks, sh).bin << kLoBits;
+    if (blockIdx.x == 0 && threadIdx.x == 0) ws->state[4] = gkey;
+  }
   __syncthreads();
-  const uint32_t gkey = ws->state[4];
   const int lane = threadIdx.x & 63;
   const int seg = blockIdx.x * (kHistThreads / 64) + (threadIdx.x >> 6);
   uint32_t* const cidx = ws->cand_idx + static_cast<int64_t>(seg) * kCandCap;
@@ -224,166 +319,83 @@ __global__ __launch_bounds__(kHistThreads) void loss_first_pass(const float* __r
   }
   const double total = block_sum<kHistThreads>(acc, smem);
   if (threadIdx.x == 0) ws->low_part[blockIdx.x] = total;
-  for (int i = threadIdx.x; i < kHiBins; i += kHistThreads)
-    if (h[i]) atomicAdd(&ws->hist_hi[i], h[i]);
+  flush_hist(h, sums, ws->hist_hi, ws->coarse_hi);  // (after block_sum's barrier)
 }
 
-// With the lists covering the threshold: zero the gradient of the listed
-// elements at or above it, and sum r^2 of the others, per list in list order.
-__global__ __launch_bounds__(kHistThreads) void loss_lists(float* __restrict__ grad, Workspace* __restrict__ ws,
-                                                           int nseg) {
-  if (!lists_serve_loss(ws)) return;
-  const uint32_t tkey = ws->state[2];
-  const int lane = threadIdx.x & 63;
-  const int seg = blockIdx.x * (kHistThreads / 64) + (threadIdx.x >> 6);
-  if (seg >= nseg) return;
-  const uint32_t* const cidx = ws->cand_idx + static_cast<int64_t>(seg) * kCandCap;
-  const float* const cr = ws->cand_r + static_cast<int64_t>(seg) * kCandCap;
-  const int cnt = static_cast<int>(ws->cand_count[seg]);  // at most kCandCap here
-  double acc = 0.0;
-  for (int j = lane; j < cnt; j += 64) {
-    const float r = cr[j];
-    if (abs_key(r) >= tkey) {
-      if (grad) grad[cidx[j]] = 0.0f;
-    } else {
-      acc += static_cast<double>(r * r);
-    }
-  }
-  for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-  if (lane == 0) ws->seg_sum[seg] = acc;
-}
-
-// Pass 2: histogram of the low 16 bits among the elements whose top 15 bits
-// are the chosen digit, straight into global memory.
-// (nseg > 0: after the fused first pass; when its lists cover the chosen bin,
-// the histogram is formed from the lists, a wave per list.)
+// Pass 2: the digit holding the k-th largest, and the histogram of the low 16
+// bits among the elements whose top 15 bits are that digit, straight into
+// global memory (its 256-bin sums by way of LDS): from the candidate lists, a
+// wave per list, when they cover the digit, else from every element.
 __global__ __launch_bounds__(kHistThreads) void radix_hist_lo(const float* __restrict__ pred,
                                                               const float* __restrict__ target,
                                                               int64_t n, Workspace* __restrict__ ws,
-                                                              int nseg) {
-  const uint32_t digit = ws->state[0];
-  if (nseg > 0 && lists_cover(ws)) {
-    const int seg = blockIdx.x * (kHistThreads / 64) + (threadIdx.x >> 6);
-    if (seg >= nseg) return;
-    const float* const cr = ws->cand_r + static_cast<int64_t>(seg) * kCandCap;
-    const int cnt = static_cast<int>(ws->cand_count[seg]);
-    for (int j = threadIdx.x & 63; j < cnt; j += 64) {
-      const uint32_t key = abs_key(cr[j]);
-      if ((key >> kLoBits) == digit) atomicAdd(&ws->hist_lo[key & (kLoBins - 1)], 1u);
-    }
-    return;
+                                                              uint32_t k, int nseg) {
+  __shared__ uint32_t sh[2];
+  __shared__ uint32_t sums[kLoBins / 256];
+  if (threadIdx.x < kLoBins / 256) sums[threadIdx.x] = 0;
+  const Picked p = pick<2, kCopies>(&ws->coarse_hi[0][0], ws->hist_hi, k, sh);
+  const uint32_t digit = p.bin;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    ws->state[0] = digit;
+    ws->state[1] = k - p.above;
   }
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * kHistThreads;
-  const int64_t first = static_cast<int64_t>(blockIdx.x) * kHistThreads + threadIdx.x;
-  auto one = [&](float r) {
-    const uint32_t key = abs_key(r);
-    if ((key >> kLoBits) == digit) {
-      // lanes sharing one key (ties, the common case among few matches)
-      // add once: keeps a degenerate input from serialising on one address
-      const uint32_t k0 = __builtin_amdgcn_readfirstlane(key);
-      const uint64_t same = __ballot(key == k0), all = __ballot(1);
-      if (same == all) {
-        if (__lane_id() == static_cast<unsigned>(__builtin_ctzll(all)))
-          atomicAdd(&ws->hist_lo[k0 & (kLoBins - 1)], static_cast<uint32_t>(__popcll(all)));
-      } else {
-        atomicAdd(&ws->hist_lo[key & (kLoBins - 1)], 1u);
+  auto count = [&](uint32_t key, uint32_t c) {
+    const uint32_t b = key & (kLoBins - 1);
+    atomicAdd(&ws->hist_lo[b], c);
+    atomicAdd(&sums[b >> 8], c);
+  };
+  if (lists_cover(ws, digit)) {
+    const int seg = blockIdx.x * (kHistThreads / 64) + (threadIdx.x >> 6);
+    if (seg < nseg) {
+      const float* const cr = ws->cand_r + static_cast<int64_t>(seg) * kCandCap;
+      const int cnt = static_cast<int>(ws->cand_count[seg]);
+      for (int j = threadIdx.x & 63; j < cnt; j += 64) {
+        const uint32_t key = abs_key(cr[j]);
+        if ((key >> kLoBits) == digit) count(key, 1u);
       }
     }
-  };
-  if ((n & 3) == 0) {
-    const float4* p4 = reinterpret_cast<const float4*>(pred);
-    const float4* t4 = reinterpret_cast<const float4*>(target);
-    for (int64_t i = first; i < n / 4; i += stride) {
-      const float4 p = p4[i], q = t4[i];
-      one(p.x - q.x);
-      one(p.y - q.y);
-      one(p.z - q.z);
-      one(p.w - q.w);
-    }
   } else {
-    for (int64_t i = first; i < n; i += stride) one(pred[i] - target[i]);
-  }
-}
-
-// The bin holding the k-th largest key: the largest b with
-// count(bins > b) < k <= count(bins >= b). One block; thread t owns the
-// per = nbins / kSelThreads consecutive bins starting at t * per (read as
-// 16-byte vectors). A suffix sum over the threads finds the owner of that
-// bin; one wave then scans the owner's bins, a lane per bin. Pass 1 records
-// the digit and the rank left inside its bin; pass 2 forms the final key;
-// the sample select (hi = 2, rank ks, at most the sample count) the guess,
-// the lower edge of the bin.
-__global__ __launch_bounds__(kSelThreads) void radix_select(int hi, Workspace* ws,
-                                                            float* __restrict__ threshold_out,
-                                                            uint32_t ks) {
-  __shared__ uint32_t wave_total[kSelThreads / 64];
-  __shared__ uint32_t win[2];  // owner thread, count strictly above its bins
-  const uint32_t* hist = hi == 2 ? ws->hist_s : hi ? ws->hist_hi : ws->hist_lo;
-  const int per = (hi ? kHiBins : kLoBins) / kSelThreads;  // 32 or 64
-  const int t = threadIdx.x;
-  const uint4* h4 = reinterpret_cast<const uint4*>(hist + t * per);
-  uint32_t mine = 0;
-  for (int j = 0; j < per / 4; ++j) {
-    const uint4 v = h4[j];
-    mine += v.x + v.y + v.z + v.w;
-  }
-  // suffix sums over threads: within each wave by shuffles, then the totals
-  // of the waves above (integer sums, so the order does not matter)
-  uint32_t above = mine;
-  const int lane_t = t & 63, wave_t = t >> 6;
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t v = __shfl_down(above, off, 64);
-    if (lane_t + off < 64) above += v;
-  }
-  if (lane_t == 0) wave_total[wave_t] = above;
-  __syncthreads();
-  for (int w = wave_t + 1; w < kSelThreads / 64; ++w) above += wave_total[w];
-  const uint32_t k = hi == 2 ? ks : ws->state[1];
-  const uint32_t run0 = above - mine;  // strictly above thread t's bins
-  if (run0 < k && k <= run0 + mine) {
-    win[0] = static_cast<uint32_t>(t);
-    win[1] = run0;
-  }
-  __syncthreads();
-  if (t >= 64) return;
-  // wave 0: lane l holds bin win[0] * per + l; suffix sums over the lanes
-  const int lane = t;
-  const int b = static_cast<int>(win[0]) * per + lane;
-  const uint32_t c = lane < per ? hist[b] : 0u;
-  uint32_t suf = c;
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t v = __shfl_down(suf, off, 64);
-    if (lane + off < 64) suf += v;
-  }
-  const uint32_t above_b = win[1] + suf - c;  // count in bins > b
-  if (lane < per && above_b < k && k <= above_b + c) {
-    if (hi == 2) {
-      ws->state[4] = static_cast<uint32_t>(b) << kLoBits;
-    } else if (hi) {
-      ws->state[0] = static_cast<uint32_t>(b);
-      ws->state[1] = k - above_b;
+    const int64_t stride = static_cast<int64_t>(gridDim.x) * kHistThreads;
+    const int64_t first = static_cast<int64_t>(blockIdx.x) * kHistThreads + threadIdx.x;
+    auto one = [&](float r) {
+      const uint32_t key = abs_key(r);
+      if ((key >> kLoBits) == digit) {
+        // lanes sharing one key (ties, the common case among few matches)
+        // add once: keeps a degenerate input from serialising on one address
+        const uint32_t k0 = __builtin_amdgcn_readfirstlane(key);
+        const uint64_t same = __ballot(key == k0), all = __ballot(1);
+        if (same == all) {
+          if (__lane_id() == static_cast<unsigned>(__builtin_ctzll(all))) count(k0, static_cast<uint32_t>(__popcll(all)));
+        } else {
+          count(key, 1u);
+        }
+      }
+    };
+    if ((n & 3) == 0) {
+      const float4* p4 = reinterpret_cast<const float4*>(pred);
+      const float4* t4 = reinterpret_cast<const float4*>(target);
+      for (int64_t i = first; i < n / 4; i += stride) {
+        const float4 a = p4[i], q = t4[i];
+        one(a.x - q.x);
+        one(a.y - q.y);
+        one(a.z - q.z);
+        one(a.w - q.w);
+      }
     } else {
-      const uint32_t key = (ws->state[0] << kLoBits) | static_cast<uint32_t>(b);
-      ws->state[2] = key;
-      if (threshold_out) *threshold_out = __uint_as_float(key);
+      for (int64_t i = first; i < n; i += stride) one(pred[i] - target[i]);
     }
   }
+  __syncthreads();
+  if (threadIdx.x < kLoBins / 256 && sums[threadIdx.x]) atomicAdd(&ws->coarse_lo[threadIdx.x], sums[threadIdx.x]);
 }
 
-// Loss and gradient. keep = |r| < threshold when a threshold is given.
-// (after_lists: the fused first pass ran; nothing to do when its lists serve.)
-__global__ __launch_bounds__(kBlock) void loss_pass(const float* __restrict__ pred,
-                                                    const float* __restrict__ target, int64_t n,
-                                                    float grad_scale, const float* __restrict__ thr_in,
-                                                    const Workspace* __restrict__ thr_ws, int use_thr,
-                                                    float* __restrict__ grad, Workspace* __restrict__ ws,
-                                                    int after_lists) {
-  if (after_lists && lists_serve_loss(ws)) return;
-  __shared__ double smem[kBlock / 64];
-  float thr = 0.0f;
-  if (use_thr) thr = thr_in ? *thr_in : __uint_as_float(thr_ws->state[2]);
+// Loss and gradient over every element by blocks 0 .. blocks - 1: keep = |r| < thr
+// with use_thr.
+__device__ __forceinline__ void full_pass(const float* __restrict__ pred, const float* __restrict__ target, int64_t n,
+                                          float grad_scale, float thr, bool use_thr, float* __restrict__ grad,
+                                          Workspace* __restrict__ ws, int blocks, double* smem) {
   double acc = 0.0;
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * kBlock;
+  const int64_t stride = static_cast<int64_t>(blocks) * kBlock;
   const bool vec = (n % 4) == 0;
   if (vec) {
     const int64_t n4 = n / 4;
@@ -416,6 +428,54 @@ __global__ __launch_bounds__(kBlock) void loss_pass(const float* __restrict__ pr
   if (threadIdx.x == 0) ws->partial[blockIdx.x] = total;
 }
 
+__global__ __launch_bounds__(kBlock) void loss_pass(const float* __restrict__ pred,
+                                                    const float* __restrict__ target, int64_t n,
+                                                    float grad_scale, const float* __restrict__ thr_in,
+                                                    float* __restrict__ grad, Workspace* __restrict__ ws) {
+  __shared__ double smem[kBlock / 64];
+  full_pass(pred, target, n, grad_scale, thr_in ? *thr_in : 0.0f, thr_in != nullptr, grad, ws, gridDim.x, smem);
+}
+
+// After the fused first pass: the threshold from the low-bits histogram; then,
+// with the lists covering it, the gradient of the listed elements at or above
+// it zeroed and r^2 of the others summed, per list in list order, a wave a
+// list; else loss and gradient by a pass over every element (`blocks` blocks).
+__global__ __launch_bounds__(kBlock) void loss_rest(const float* __restrict__ pred, const float* __restrict__ target,
+                                                    int64_t n, float grad_scale, float* __restrict__ grad,
+                                                    Workspace* __restrict__ ws, float* __restrict__ threshold_out,
+                                                    int nseg, int blocks) {
+  __shared__ double smem[kBlock / 64];
+  __shared__ uint32_t sh[2];
+  const uint32_t digit = ws->state[0];
+  const uint32_t tkey = (digit << kLoBits) | pick<4, 1>(ws->coarse_lo, ws->hist_lo, ws->state[1], sh).bin;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    ws->state[2] = tkey;
+    if (threshold_out) *threshold_out = __uint_as_float(tkey);
+  }
+  if (!lists_serve_loss(ws, digit, tkey)) {
+    if (static_cast<int>(blockIdx.x) < blocks)
+      full_pass(pred, target, n, grad_scale, __uint_as_float(tkey), true, grad, ws, blocks, smem);
+    return;
+  }
+  const int lane = threadIdx.x & 63;
+  const int seg = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+  if (seg >= nseg) return;
+  const uint32_t* const cidx = ws->cand_idx + static_cast<int64_t>(seg) * kCandCap;
+  const float* const cr = ws->cand_r + static_cast<int64_t>(seg) * kCandCap;
+  const int cnt = static_cast<int>(ws->cand_count[seg]);  // at most kCandCap here
+  double acc = 0.0;
+  for (int j = lane; j < cnt; j += 64) {
+    const float r = cr[j];
+    if (abs_key(r) >= tkey) {
+      if (grad) grad[cidx[j]] = 0.0f;
+    } else {
+      acc += static_cast<double>(r * r);
+    }
+  }
+  for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+  if (lane == 0) ws->seg_sum[seg] = acc;
+}
+
 // (nseg > 0: after the fused first pass; when its lists serve, the loss is
 // the first pass's block sums plus the lists' sums.)
 __global__ __launch_bounds__(kBlock) void finalize(const Workspace* __restrict__ ws, int nparts,
@@ -424,7 +484,7 @@ __global__ __launch_bounds__(kBlock) void finalize(const Workspace* __restrict__
   __shared__ double smem[kBlock / 64];
   double acc = 0.0;
   // Fixed assignment of partials to threads and a fixed tree: deterministic.
-  if (nseg > 0 && lists_serve_loss(ws)) {
+  if (nseg > 0 && lists_serve_loss(ws, ws->state[0], ws->state[2])) {
     for (int i = threadIdx.x; i < nlow; i += kBlock) acc += ws->low_part[i];
     for (int i = threadIdx.x; i < nseg; i += kBlock) acc += ws->seg_sum[i];
   } else {
@@ -476,29 +536,27 @@ int outlier(const char* fn, const float* pred, const float* target, int64_t n, i
     // the guess: rank 2 ceil(k / 37) + 64 among the samples (none when the sample is smaller)
     const int64_t ns = sample_count(n);
     const int64_t ks = 2 * ((k + kSampleStride - 1) / kSampleStride) + 64;
+    uint32_t guess = 0;
     if (ks <= ns) {
       const int64_t sg = ns / kHistThreads + 1;
       hipLaunchKernelGGL(sample_hist, dim3(static_cast<unsigned>(sg < kHistBlocks ? sg : kHistBlocks)),
                          dim3(kHistThreads), 0, s, pred, target, n, ws);
-      hipLaunchKernelGGL(radix_select, dim3(1), dim3(kSelThreads), 0, s, 2, ws, nullptr,
-                         static_cast<uint32_t>(ks));
+      guess = static_cast<uint32_t>(ks);
     }
     hipLaunchKernelGGL(loss_first_pass, dim3(hist_grid), dim3(kHistThreads), 0, s, pred, target, n, gscale,
-                       grad_out, ws);
-    hipLaunchKernelGGL(radix_select, dim3(1), dim3(kSelThreads), 0, s, 1, ws, threshold_out, 0u);
-    hipLaunchKernelGGL(radix_hist_lo, dim3(hist_grid), dim3(kHistThreads), 0, s, pred, target, n, ws, nseg);
-    hipLaunchKernelGGL(radix_select, dim3(1), dim3(kSelThreads), 0, s, 0, ws, threshold_out, 0u);
-    hipLaunchKernelGGL(loss_lists, dim3(hist_grid), dim3(kHistThreads), 0, s, grad_out, ws, nseg);
-    hipLaunchKernelGGL(loss_pass, dim3(grid), dim3(kBlock), 0, s, pred, target, n, gscale, nullptr, ws, 1,
-                       grad_out, ws, 1);
+                       grad_out, ws, guess);
+    hipLaunchKernelGGL(radix_hist_lo, dim3(hist_grid), dim3(kHistThreads), 0, s, pred, target, n, ws,
+                       static_cast<uint32_t>(k), nseg);
+    const int list_grid = nseg / (kBlock / 64);
+    hipLaunchKernelGGL(loss_rest, dim3(grid > list_grid ? grid : list_grid), dim3(kBlock), 0, s, pred, target, n, gscale,
+                       grad_out, ws, threshold_out, nseg, grid);
     hipLaunchKernelGGL(finalize, dim3(1), dim3(kBlock), 0, s, ws, grid, static_cast<double>(denom), loss_out,
                        hist_grid, nseg);
     MR_LAUNCH_CHECK(fn);
     return MR_OK;
   }
   if (threshold_out) return fail(MR_EINVAL, "%s: threshold_out is only written when it is computed", fn);
-  hipLaunchKernelGGL(loss_pass, dim3(grid), dim3(kBlock), 0, s, pred, target, n, gscale,
-                     threshold_in, ws, 1, grad_out, ws, 0);
+  hipLaunchKernelGGL(loss_pass, dim3(grid), dim3(kBlock), 0, s, pred, target, n, gscale, threshold_in, grad_out, ws);
   hipLaunchKernelGGL(finalize, dim3(1), dim3(kBlock), 0, s, ws, grid, static_cast<double>(denom),
                      loss_out, 0, 0);
   MR_LAUNCH_CHECK(fn);
@@ -510,7 +568,7 @@ int outlier(const char* fn, const float* pred, const float* target, int64_t n, i
 
 // The allocation-free outlier loss keeps its workspace in this array, one
 // copy per GPU, held until the process ends (kScratchBytes = the Workspace,
-// 4,778,016 bytes). Host code never passes the array's name to a kernel: that
+// 4,787,232 bytes). Host code never passes the array's name to a kernel: that
 // name is a host-side stand-in. The device address comes from
 // hipGetSymbolAddress, once per device, on the first call there.
 static __device__ __align__(256) unsigned char scratch[mr::kScratchBytes];
@@ -560,8 +618,7 @@ int mr_loss_mse(const float* pred, const float* target, int64_t n, int64_t denom
   Workspace* ws = static_cast<Workspace*>(workspace);
   const int grid = grid_for(n);
   const float gscale = static_cast<float>(2.0 / static_cast<double>(denom));
-  hipLaunchKernelGGL(loss_pass, dim3(grid), dim3(kBlock), 0, s, pred, target, n, gscale, nullptr,
-                     nullptr, 0, grad_out, ws, 0);
+  hipLaunchKernelGGL(loss_pass, dim3(grid), dim3(kBlock), 0, s, pred, target, n, gscale, nullptr, grad_out, ws);
   hipLaunchKernelGGL(finalize, dim3(1), dim3(kBlock), 0, s, ws, grid, static_cast<double>(denom),
                      loss_out, 0, 0);
   MR_LAUNCH_CHECK("mr_loss_mse");
