@@ -11,15 +11,17 @@
 // bit-identical to a float32 evaluation of the reference's formulas; only the
 // per-group sums of the backward differ, by summation order.
 //
-// Two launch shapes:
+// Three launch shapes:
 //   fast    each lane owns 8 consecutive weights; a group of gs weights spans
 //           gs/8 adjacent lanes (a power of two <= 64) and its min/max and
 //           gradient sums are xor-butterfly reductions over those lanes, so
 //           every lane of the group ends with bit-identical group values.
 //           One wave streams 8 * 64 weights with 16-byte loads: W, v and the
 //           outputs are read and written exactly once (HBM-bound).
-//   generic one wave per group, strided over the group; covers per-channel
-//           groups, padded last groups and fp16 inputs.
+//   row     64, 256 or 1024 threads hold a whole long group in registers, 8
+//           consecutive weights at a time (per-channel groups).
+//   generic one wave per group, strided over the group, rereading it for each
+//           pass; covers padded last groups and odd sizes.
 #include <cmath>
 
 #include "mr_common.h"
@@ -798,12 +800,255 @@ __global__ __launch_bounds__(kBlock) void fq_bwd_generic(
   }
 }
 
+// -------------------------------------------------- long groups in registers --
+//
+// Per-channel groups (one scale a row) and other groups of 256 weights and
+// more that are not 8 * 2^k: T threads (a wave, four or sixteen) own a group, each
+// up to kRowChunks runs of 8 consecutive weights, so that W, v and the gradient
+// are read once, in 16-byte loads, before the extremes are known, and the
+// backward's sums need no second read. HBM-bound. The wave-per-group form
+// read each operand two or three times, 2 or 4 bytes a lane: measured on a
+// float16 4864 x 896 weight with one group a row, forward 21 and fused step 23
+// us, 8 and 16 here (3.5 and 4.7 TB/s past the launch). (Two runs a thread for
+// the shorter groups, half the registers, measured the same.)
+constexpr int kRowChunks = 4;
+
+__device__ __forceinline__ void load8_any(const void* p, int dt, int64_t e, float (&x)[8]) {
+  if (dt == MR_BF16) load8<MR_BF16>(p, e, x);
+  else if (dt == MR_F16) load8<MR_F16>(p, e, x);
+  else load8<MR_F32>(p, e, x);
+}
+__device__ __forceinline__ void store8_any(void* p, int dt, int64_t e, const float (&x)[8]) {
+  if (dt == MR_BF16) store8<MR_BF16>(p, e, x);
+  else if (dt == MR_F16) store8<MR_F16>(p, e, x);
+  else store8<MR_F32>(p, e, x);
+}
+
+// w / s of 8 weights, correctly rounded (see quotients()); mx, mn: the group's extremes.
+template <int MODE>
+__device__ __forceinline__ void row_quotients(const float (&x)[8], int wt, float s, float mx, float mn, float (&t)[8]) {
+  if (wt == MR_BF16) {
+    quotients<MR_BF16, MODE>(x, s, lane_quotients_fast<MR_BF16>(x, mx, mn), t);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) t[k] = x[k] / s;
+  }
+}
+
+// OP over the T threads of a group; every thread gets the result. `sm`: a word
+// per wave of the block (unused by a single wave).
+template <int T, typename OP>
+__device__ __forceinline__ float row_reduce(float x, float* sm, OP op) {
+  for (int off = 32; off > 0; off >>= 1) x = op(x, __shfl_xor(x, off, 64));
+  if constexpr (T > 64) {
+    __syncthreads();  // (an earlier reduction's words have been read)
+    if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = x;
+    __syncthreads();
+    x = sm[0];
+    for (int i = 1; i < T / 64; ++i) x = op(x, sm[i]);
+  }
+  return x;
+}
+
+// The group of this thread, and the thread's index in it.
+template <int T>
+__device__ __forceinline__ int64_t row_group(int& t) {
+  if constexpr (T == 64) {
+    t = threadIdx.x & 63;
+    return static_cast<int64_t>(blockIdx.x) * (kBlock / 64) + (threadIdx.x >> 6);
+  }
+  t = threadIdx.x;
+  return blockIdx.x;
+}
+
+template <int MODE, int T>
+__device__ __forceinline__ void row_extremes(const float (&x)[kRowChunks][8], int nc, int t, float* sm, float& mx, float& mn) {
+  mx = mn = 0.0f;  // (the extremes are taken with zero)
+  if constexpr (MODE != MR_SYM_SEARCHED) {
+#pragma unroll
+    for (int k = 0; k < kRowChunks; ++k) {
+      if (t + k * T >= nc) continue;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        mx = fmaxf(mx, x[k][j]);
+        mn = fminf(mn, x[k][j]);
+      }
+    }
+    mx = row_reduce<T>(mx, sm, [](float a, float b) { return fmaxf(a, b); });
+    mn = row_reduce<T>(mn, sm, [](float a, float b) { return fminf(a, b); });
+  }
+}
+
+template <int MODE, bool HAS_V, int T>
+__global__ __launch_bounds__(T == 64 ? kBlock : T) void fq_fwd_row(
+    const void* __restrict__ w, int wt, const float* __restrict__ v, const float* __restrict__ alpha,
+    const float* __restrict__ beta, const float* __restrict__ init_scale, void* __restrict__ wq, int ot,
+    uint8_t* __restrict__ codes, float* __restrict__ scale_out, float* __restrict__ zp_out, int64_t n_groups,
+    int64_t cols, int gs, int64_t ng, float maxq, float inv_maxq, float qmin, float qmax, float eps, RowMap map) {
+  __shared__ float sm[16];
+  int t;
+  const int64_t grp = row_group<T>(t);
+  if (grp >= n_groups) return;  // (whole waves, and only where no barrier follows)
+  const int nc = gs / 8;
+  float x[kRowChunks][8], vv[kRowChunks][8];
+#pragma unroll
+  for (int k = 0; k < kRowChunks; ++k) {
+    const int c = t + k * T;
+    if (c >= nc) continue;
+    load8_any(w, wt, grp * gs + c * 8, x[k]);
+    if constexpr (HAS_V) load8_f32_cached(v, grp * gs + c * 8, vv[k]);
+  }
+  float mx, mn;
+  row_extremes<MODE, T>(x, nc, t, sm, mx, mn);
+  float a = 1.0f, b = 1.0f, base = 0.0f;
+  if constexpr (HAS_V) {
+    a = alpha[grp];
+    b = beta[grp];
+  }
+  if constexpr (MODE == MR_SYM_SEARCHED) base = init_scale[grp];
+  const Group p = group_params<MODE>(mx, mn, a, b, base, maxq, inv_maxq, eps);
+  const int64_t out = wq ? map.row(grp / ng) * cols + (grp % ng) * gs : 0;
+#pragma unroll
+  for (int k = 0; k < kRowChunks; ++k) {
+    const int c = t + k * T;
+    if (c >= nc) continue;
+    float lmx = mx, lmn = mn;
+    if constexpr (MODE == MR_SYM_SEARCHED) {  // (no group extremes: the lane's own bound its quotients)
+      lmx = lmn = x[k][0];
+#pragma unroll
+      for (int j = 1; j < 8; ++j) {
+        lmx = fmaxf(lmx, x[k][j]);
+        lmn = fminf(lmn, x[k][j]);
+      }
+    }
+    float q[8], code[8], tq[8];
+    row_quotients<MODE>(x[k], wt, p.s, lmx, lmn, tq);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      float in;
+      q[j] = quant_t<MODE, HAS_V>(tq[j], HAS_V ? vv[k][j] : 0.0f, p, qmin, qmax, code[j], in);
+    }
+    if (wq) store8_any(wq, ot, out + c * 8, q);
+    if (codes) {
+      uint32_t lo = 0, hi = 0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        lo |= (static_cast<uint32_t>(static_cast<int>(code[j])) & 0xffu) << (8 * j);
+        hi |= (static_cast<uint32_t>(static_cast<int>(code[j + 4])) & 0xffu) << (8 * j);
+      }
+      *reinterpret_cast<uint2*>(codes + grp * gs + c * 8) = make_uint2(lo, hi);
+    }
+  }
+  if (t == 0) {
+    if (scale_out) scale_out[grp] = p.s;
+    if (zp_out) zp_out[grp] = p.zp;
+  }
+}
+
+template <int MODE, bool UPDATE, int T>
+__global__ __launch_bounds__(T == 64 ? kBlock : T) void fq_bwd_row(
+    const void* __restrict__ w, int wt, float* __restrict__ v, float* __restrict__ alpha, float* __restrict__ beta,
+    const float* __restrict__ init_scale, const void* __restrict__ g, int gt, int64_t n_groups, int64_t cols, int gs,
+    int64_t ng, float maxq, float inv_maxq, float qmin, float qmax, float eps, StepArgs st, float* __restrict__ gv_out,
+    float* __restrict__ ga_out, float* __restrict__ gb_out, RowMap map) {
+  __shared__ float sm[16];
+  if constexpr (UPDATE) st.lr = st.rate();
+  int t;
+  const int64_t grp = row_group<T>(t);
+  if (grp >= n_groups) return;
+  const int nc = gs / 8;
+  const int64_t placed = map.row(grp / ng) * cols + (grp % ng) * gs;
+  float x[kRowChunks][8], vv[kRowChunks][8], gg[kRowChunks][8];
+#pragma unroll
+  for (int k = 0; k < kRowChunks; ++k) {
+    const int c = t + k * T;
+    if (c >= nc) continue;
+    load8_any(w, wt, grp * gs + c * 8, x[k]);
+    load8_f32_cached(v, grp * gs + c * 8, vv[k]);
+    load8_any(g, gt, placed + c * 8, gg[k]);
+  }
+  float mx, mn;
+  row_extremes<MODE, T>(x, nc, t, sm, mx, mn);
+  const float a = alpha[grp], b = beta[grp];
+  float base = 0.0f;
+  if constexpr (MODE == MR_SYM_SEARCHED) base = init_scale[grp];
+  const Group p = group_params<MODE>(mx, mn, a, b, base, maxq, inv_maxq, eps);
+  auto lane_bounds = [&](int k, float& lmx, float& lmn) __attribute__((always_inline)) {
+    lmx = mx;
+    lmn = mn;
+    if constexpr (MODE == MR_SYM_SEARCHED) {
+      lmx = lmn = x[k][0];
+#pragma unroll
+      for (int j = 1; j < 8; ++j) {
+        lmx = fmaxf(lmx, x[k][j]);
+        lmn = fminf(lmn, x[k][j]);
+      }
+    }
+  };
+  float sum_s = 0.0f, sum_d = 0.0f;
+#pragma unroll
+  for (int k = 0; k < kRowChunks; ++k) {
+    const int c = t + k * T;
+    if (c >= nc) continue;
+    float lmx, lmn, tq[8];
+    lane_bounds(k, lmx, lmn);
+    row_quotients<MODE>(x[k], wt, p.s, lmx, lmn, tq);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const BwdTerms<MODE> tm = bwd_one<MODE>(tq[j], vv[k][j], gg[k][j], p, p.wmin_s, qmin, qmax);
+      sum_s = sum_s + tm.ts;
+      if constexpr (MODE == MR_ASYM) sum_d = sum_d + tm.td;
+      gg[k][j] = tm.gv;  // the gradient of v from here on
+    }
+    if (gv_out) store8_f32(gv_out, grp * gs + c * 8, gg[k]);
+    if constexpr (UPDATE) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) vv[k][j] = clampf(vv[k][j] - st.lr * signf(gg[k][j]), -st.vb, st.vb);
+      store8_f32_cached(v, grp * gs + c * 8, vv[k]);
+    }
+  }
+  auto add = [](float p1, float p2) { return p1 + p2; };
+  sum_s = row_reduce<T>(sum_s, sm, add);
+  if constexpr (MODE == MR_ASYM) sum_d = row_reduce<T>(sum_d, sm, add);
+  float ga, gb;
+  coef_grads<MODE>(p, sum_s, sum_d, maxq, ga, gb);
+  if (t == 0) {
+    if (ga_out) ga_out[grp] = ga;
+    if (gb_out) gb_out[grp] = gb;
+  }
+  if constexpr (UPDATE) {
+    const float na = clampf(a - st.lr * signf(ga), st.lo, st.hi);
+    const float nb = clampf(b - st.lr * signf(gb), st.lo, st.hi);
+    if (t == 0) {  // (every thread read a and b ahead of the reductions' barriers, or in this wave's order)
+      alpha[grp] = na;
+      beta[grp] = nb;
+    }
+    if (st.wq) {
+      const Group p2 = group_params<MODE>(mx, mn, na, nb, base, maxq, inv_maxq, eps);
+#pragma unroll
+      for (int k = 0; k < kRowChunks; ++k) {
+        const int c = t + k * T;
+        if (c >= nc) continue;
+        float lmx, lmn, tq[8], q[8];
+        lane_bounds(k, lmx, lmn);
+        row_quotients<MODE>(x[k], wt, p2.s, lmx, lmn, tq);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          float code, in;
+          q[j] = quant_t<MODE, true>(tq[j], vv[k][j], p2, qmin, qmax, code, in);
+        }
+        store8_any(st.wq, st.wq_dt, placed + c * 8, q);
+      }
+    }
+  }
+}
+
 // ------------------------------------------------------------ host side --
 
 struct Shape {
   int64_t rows, cols, ng, n_groups;
   int gs, tpg, tpg_shift;
-  bool fast;
+  bool fast, row;  // row: whole groups of 256 .. 32768 weights, a multiple of 8, held by row_threads()
   float maxq, inv_maxq, qmin, qmax;  // inv_maxq = RN(1 / maxq)
 };
 
@@ -832,6 +1077,7 @@ int check_common(const char* fn, const void* w, int w_dtype, int64_t rows, int64
   sh.tpg_shift = 0;
   while (pow2 && (1 << sh.tpg_shift) < tpg) ++sh.tpg_shift;
   sh.fast = (sh.gs % 8 == 0) && pow2 && gs > 0 && (cols % gs == 0);
+  sh.row = gs >= 256 && gs <= 1024 * 8 * kRowChunks && gs % 8 == 0 && cols % gs == 0;
   if (mode == MR_ASYM) {
     sh.maxq = static_cast<float>((1 << bits) - 1);
     sh.qmin = 0.0f;
@@ -845,12 +1091,17 @@ int check_common(const char* fn, const void* w, int w_dtype, int64_t rows, int64
   return MR_OK;
 }
 
+// Threads per group of the row kernels: the fewest whose registers hold it.
+int row_threads(int gs) {
+  return gs <= 64 * 8 * kRowChunks ? 64 : gs <= 256 * 8 * kRowChunks ? 256 : 1024;
+}
+
 template <int MODE, bool HAS_V>
 int launch_fwd(const Shape& sh, const void* w, int wt, const float* v, const float* alpha,
                const float* beta, const float* init_scale, void* wq, int ot, uint8_t* codes,
                float* scale_out, float* zp_out, float eps, RowMap map, hipStream_t stream) {
   map.prepare(sh.cols);
-  const bool fast_types = (wt == MR_F32 || wt == MR_BF16) && (!wq || ot == MR_F32 || ot == MR_BF16);
+  const bool fast_types = wt == MR_F16 || !wq || ot == MR_F32 || ot == MR_BF16;
   const bool fast_align = aligned16(w) && (!HAS_V || aligned16(v)) && (!wq || aligned16(wq)) &&
                           (!codes || (reinterpret_cast<uintptr_t>(codes) & 7u) == 0);
   if (sh.fast && fast_types && fast_align) {
@@ -870,12 +1121,28 @@ int launch_fwd(const Shape& sh, const void* w, int wt, const float* v, const flo
     else MR_FWD_FAST_T(WT_, OT_, 0);                                        \
   } while (0)
     const int o = wq ? ot : MR_F32;
-    if (wt == MR_BF16 && o == MR_BF16) MR_FWD_FAST(MR_BF16, MR_BF16);
+    // (fp16 weights: one group-width form, quotients by division)
+    if (wt == MR_F16 && o == MR_F16) MR_FWD_FAST_T(MR_F16, MR_F16, 0);
+    else if (wt == MR_F16 && o == MR_BF16) MR_FWD_FAST_T(MR_F16, MR_BF16, 0);
+    else if (wt == MR_F16) MR_FWD_FAST_T(MR_F16, MR_F32, 0);
+    else if (wt == MR_BF16 && o == MR_BF16) MR_FWD_FAST(MR_BF16, MR_BF16);
     else if (wt == MR_BF16) MR_FWD_FAST(MR_BF16, MR_F32);
     else if (o == MR_BF16) MR_FWD_FAST(MR_F32, MR_BF16);
     else MR_FWD_FAST(MR_F32, MR_F32);
 #undef MR_FWD_FAST_T
 #undef MR_FWD_FAST
+  } else if (sh.row && fast_align) {
+    const int T = row_threads(sh.gs);
+    const int64_t blocks = T == 64 ? (sh.n_groups + 3) / 4 : sh.n_groups;
+    if (blocks > 0x7fffffff) return fail(MR_EINVAL, "mr_fq_forward: tensor too large");
+#define MR_FWD_ROW(T_)                                                                                         \
+  hipLaunchKernelGGL((fq_fwd_row<MODE, HAS_V, T_>), dim3(static_cast<unsigned>(blocks)), dim3(T_ == 64 ? kBlock : T_), \
+                     0, stream, w, wt, v, alpha, beta, init_scale, wq, ot, codes, scale_out, zp_out, sh.n_groups,  \
+                     sh.cols, sh.gs, sh.ng, sh.maxq, sh.inv_maxq, sh.qmin, sh.qmax, eps, map)
+    if (T == 64) MR_FWD_ROW(64);
+    else if (T == 256) MR_FWD_ROW(256);
+    else MR_FWD_ROW(1024);
+#undef MR_FWD_ROW
   } else {
     const int64_t blocks = (sh.n_groups + 3) / 4;
     if (blocks > 0x7fffffff) return fail(MR_EINVAL, "mr_fq_forward: tensor too large");
@@ -893,7 +1160,7 @@ int launch_bwd(const Shape& sh, const void* w, int wt, float* v, float* alpha, f
                const float* init_scale, const void* g, int gt, float eps, StepArgs st,
                float* gv_out, float* ga_out, float* gb_out, RowMap map, hipStream_t stream) {
   map.prepare(sh.cols);
-  const bool fast_types = (wt == MR_F32 || wt == MR_BF16) && (gt == MR_F32 || gt == MR_BF16);
+  const bool fast_types = gt == MR_F32 || gt == MR_BF16;
   const bool fast_align = aligned16(w) && aligned16(v) && aligned16(g) && (!gv_out || aligned16(gv_out));
   if (sh.fast && fast_types && fast_align) {
     const int64_t n_chunks = sh.rows * sh.cols / 8;
@@ -911,12 +1178,26 @@ int launch_bwd(const Shape& sh, const void* w, int wt, float* v, float* alpha, f
     else if (sh.tpg == 16) MR_BWD_FAST_T(WT_, GT_, 16);                     \
     else MR_BWD_FAST_T(WT_, GT_, 0);                                        \
   } while (0)
-    if (wt == MR_BF16 && gt == MR_F32) MR_BWD_FAST(MR_BF16, MR_F32);
+    if (wt == MR_F16 && gt == MR_F32) MR_BWD_FAST_T(MR_F16, MR_F32, 0);
+    else if (wt == MR_F16) MR_BWD_FAST_T(MR_F16, MR_BF16, 0);
+    else if (wt == MR_BF16 && gt == MR_F32) MR_BWD_FAST(MR_BF16, MR_F32);
     else if (wt == MR_BF16) MR_BWD_FAST(MR_BF16, MR_BF16);
     else if (gt == MR_F32) MR_BWD_FAST(MR_F32, MR_F32);
     else MR_BWD_FAST(MR_F32, MR_BF16);
 #undef MR_BWD_FAST_T
 #undef MR_BWD_FAST
+  } else if (sh.row && fast_align) {
+    const int T = row_threads(sh.gs);
+    const int64_t blocks = T == 64 ? (sh.n_groups + 3) / 4 : sh.n_groups;
+    if (blocks > 0x7fffffff) return fail(MR_EINVAL, "mr_fq_backward_signsgd: tensor too large");
+#define MR_BWD_ROW(T_)                                                                                         \
+  hipLaunchKernelGGL((fq_bwd_row<MODE, UPDATE, T_>), dim3(static_cast<unsigned>(blocks)), dim3(T_ == 64 ? kBlock : T_), \
+                     0, stream, w, wt, v, alpha, beta, init_scale, g, gt, sh.n_groups, sh.cols, sh.gs, sh.ng, sh.maxq, \
+                     sh.inv_maxq, sh.qmin, sh.qmax, eps, st, gv_out, ga_out, gb_out, map)
+    if (T == 64) MR_BWD_ROW(64);
+    else if (T == 256) MR_BWD_ROW(256);
+    else MR_BWD_ROW(1024);
+#undef MR_BWD_ROW
   } else {
     const int64_t blocks = (sh.n_groups + 3) / 4;
     if (blocks > 0x7fffffff) return fail(MR_EINVAL, "mr_fq_backward_signsgd: tensor too large");

@@ -245,3 +245,74 @@ def test_step_requant_writes_the_next_forward(shape, mode):
         mask = torch.ones(wbig.shape[0], dtype=torch.bool, device=dev())
         mask[idx] = False
         assert bool((wbig[mask] == 7.0).all())
+
+
+def _unaligned(t):
+    """The same tensor one element off its 16-byte alignment (the generic kernels' inputs)."""
+    buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    out = buf[1:].view(t.shape)
+    out.copy_(t)
+    return out
+
+
+# Long groups in registers (64, 256 and 1024 threads; the largest of each and one
+# run past it; 32776 weights are past the last) and float16 weights on both
+# aligned forms, against the oracle and, bit for bit but for the order of the
+# coefficients' sums, against the generic kernels on unaligned inputs.
+@pytest.mark.parametrize("mode", ["asym", "sym", "searched"])
+@pytest.mark.parametrize("shape", [(6, 256, -1), (5, 2048, -1), (3, 2056, -1), (3, 8200, -1), (2, 18944, -1),
+                                   (2, 32768, -1), (2, 32776, -1), (4, 1200, 600), (40, 192, 64), (24, 256, 8)])
+@pytest.mark.parametrize("wdtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_long_groups_and_float16(mode, shape, wdtype):
+    rows, cols, gs = shape
+    bits, lr = (3, 0.005) if mode == "sym" else (4, 0.003)
+    _note("long groups", mode, shape, wdtype)
+    w = weight(rows, cols, seed=cols, dtype=wdtype)
+    v, a, b = params(rows, cols, gs, seed=bits, coef_jitter=0.3)
+    g = torch.randn(rows, cols, generator=torch.Generator().manual_seed(bits)) * 1e-3
+    init = _init_scale(rows, cols, gs) if mode == "searched" else None
+    init_np, init_d = (None, None) if init is None else (init.numpy(), init.to(dev()))
+    scheme = _scheme(mode, bits, gs)
+    wn, gn = w.float().numpy(), g.numpy()
+    ref_q, ref_c, ref_s, ref_zp = oracle_fq(wn, v, a, b, bits, gs, mode, init_np)
+    ref_gv, ref_ga, ref_gb = Q.quantize_grad(wn, v.numpy(), a.numpy(), b.numpy(), gn, bits=bits, group_size=gs,
+                                             mode=mode, init_scale=init_np, dtype=np.float32)
+    ss, sd = _grad_tolerance(wn, v.numpy(), a.numpy(), b.numpy(), gn, bits, gs, mode, init_np)
+    gs_eff = cols if gs == -1 else gs
+    tol = (gs_eff / 64 + 16) * np.finfo(np.float32).eps * (ss + sd) + 1e-30
+    lo, hi = scheme.coefficient_bounds
+    seen = []
+    for place in (lambda t: t, _unaligned):
+        wd = place(w.to(dev()))
+        p = {"v": place(v.to(dev())), "alpha": a.to(dev()), "beta": b.to(dev())}
+        outs = [QZ.fake_quantize(wd, p, scheme, init_scale=init_d, out_dtype=dt)
+                for dt in (torch.float32, torch.bfloat16, torch.float16)]
+        codes, scale, zp = QZ.quantize_codes(wd, p, scheme, init_scale=init_d, narrow=True)
+        assert np.array_equal(to_np(outs[0]), ref_q) and np.array_equal(to_np(outs[1]), Q.round_to_bf16(ref_q))
+        assert np.array_equal(to_np(codes).astype(np.int64), ref_c.astype(np.int64))
+        assert np.array_equal(to_np(scale), ref_s) and (zp is None or np.array_equal(to_np(zp), ref_zp))
+        grads = QZ.quantize_grad(wd, p, scheme, g.to(dev()), init_scale=init_d)
+        assert np.array_equal(to_np(grads["v"]), ref_gv), "grad v differs"
+        assert np.all(np.abs(to_np(grads["alpha"]) - ref_ga) <= tol)
+        assert np.all(np.abs(to_np(grads["beta"]) - ref_gb) <= tol)
+        SG.fused_step(wd, p, g.to(dev()), scheme, lr, init_scale=init_d)
+        ref_v = np.clip(v.numpy() - np.float32(lr) * np.sign(ref_gv), -0.5, 0.5)
+        assert np.array_equal(to_np(p["v"]), ref_v), "updated v differs"
+        for name, ref_grad, base in (("alpha", ref_ga, a.numpy()), ("beta", ref_gb, b.numpy())):
+            clear = np.abs(ref_grad) > tol
+            assert np.array_equal(to_np(p[name])[clear], np.clip(base - np.float32(lr) * np.sign(ref_grad), lo, hi)[clear])
+        # the step that also writes W' into a placed buffer: the next forward's values
+        q = {k: place(t.to(dev())) if k == "v" else t.to(dev()) for k, t in (("v", v), ("alpha", a), ("beta", b))}
+        placed = torch.full((rows + 3, cols), 7.0, dtype=torch.float16, device=dev())
+        gp = torch.zeros(rows + 3, cols, device=dev())
+        gp[2:rows + 2] = g.to(dev())
+        from mround_amd import kernels as K
+
+        K.fq_step_requant_mapped(wd, q["v"], q["alpha"], q["beta"], gp, bits=bits, group_size=gs, mode=mode, eps=1e-8,
+                                 lr=lr, coef_lo=lo, coef_hi=hi, v_bound=0.5, row_block=rows, row_stride=rows,
+                                 row_offset=2, wq_out=placed, init_scale=init_d)
+        assert all(torch.equal(q[k], p[k]) for k in q)
+        nxt = QZ.fake_quantize(wd, p, scheme, init_scale=init_d, out_dtype=torch.float16)
+        assert torch.equal(placed[2:rows + 2], nxt) and bool((placed[:2] == 7).all()) and bool((placed[rows + 2:] == 7).all())
+        seen.append(outs[2])
+    assert torch.equal(*seen)
