@@ -158,7 +158,15 @@ def dtype_code(dtype: torch.dtype) -> int:
         raise KernelError(f"unsupported dtype {dtype}; expected float32, bfloat16 or float16") from None
 
 
+# The current stream's handle without building a Stream object: 0.1 us against
+# 2.1, of the 7 us that a call through this binding takes (4 of them the
+# launch itself).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(t: torch.Tensor) -> int:
+    if _raw_stream is not None and t.is_cuda:
+        return _raw_stream(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
