@@ -279,12 +279,14 @@ int mr_embed_rows(const void* table, int dtype, int64_t V, int64_t H, int64_t ld
  * All row-major with leading dimensions lda/ldb/ldc/ldr in elements; M, N
  * multiples of 8, K a multiple of 64, operands, C and resid 16-byte aligned
  * with rows a multiple of 16 bytes apart. C is fp32 or
- * bf16; with resid (fp32) C is fp32. Long-K problems whose 256 x 256 tiles
- * leave a partial last wave sum that remainder from k-split partial tiles in
- * the caller's workspace: mr_gemm_workspace_bytes(M, N, K) bytes (0 when the
- * shape is not split; N is the product's width, 2N for mr_gemm_swiglu), at
- * most 128 MB, 16-byte aligned. A NULL or smaller workspace narrows or
- * drops the split: the same product, summed in another order. Outputs and
+ * bf16; with resid (fp32) C is fp32. Long-K problems (and
+ * weight gradients of any K) whose tiles leave a partial last wave sum that
+ * remainder from k-split partial tiles in the caller's workspace:
+ * mr_gemm_workspace_bytes(M, N, K) bytes (0 when the shape is not split; N is
+ * the product's width, 2N for mr_gemm_swiglu), at most 128 MB, 16-byte
+ * aligned. A NULL or smaller workspace narrows or drops the split: the same
+ * product, summed in another order. With K under 6144, MR_NT and MR_NN rows
+ * are the same bits for every M. Outputs and
  * the workspace must not overlap the operands or each other (refused with
  * MR_EINVAL); C may be resid itself (same pointer and leading dimension), and
  * mr_gemm_swiglu_bwd's dgu may be its gu. Replaces the

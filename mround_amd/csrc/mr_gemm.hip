@@ -1374,8 +1374,13 @@ struct Plan {
 // 9728 x 896 x 16384, two whole rounds, 353 against 290).
 constexpr int kDeepMaxKt = 320, kDeepMaxKtRounds = 160;
 
-// The plan of an M x N x (64 KT) product with ws_bytes for partials.
-Plan plan_for(int64_t M, int64_t N, int KT, Output o, int64_t ws_bytes) {
+// The plan of an M x N x (64 KT) product with ws_bytes for partials. rows: M
+// counts activation rows (NT, NN), not weight rows (TN). There a product of
+// under kSplitMinKt k-tiles is never cut along K, so that a row's sums are the
+// same bits whatever other rows come with it: a step in pieces has the
+// activations of the whole batch's step. (Cutting them too gained 9 us of a
+// 0.5B scoring batch's 2,397.)
+Plan plan_for(int64_t M, int64_t N, int KT, bool rows, Output o, int64_t ws_bytes) {
   const int64_t big = ((M + 255) / 256) * ((N + 255) / 256);
   const int64_t small = ((M + 127) / 128) * ((N + 127) / 128);
   Plan p{BIG, 1};
@@ -1386,7 +1391,7 @@ Plan plan_for(int64_t M, int64_t N, int KT, Output o, int64_t ws_bytes) {
   }
   const int64_t tail = small % 256;
   for (int sp = 1; sp <= 16; ++sp) {
-    if (sp > 1 && (!tail || tail * sp > 256 || sp * 2 > KT || tail * sp * (128ll * 128 * 4) > ws_bytes)) break;
+    if (sp > 1 && (!tail || (rows && KT < kSplitMinKt) || tail * sp > 256 || sp * 2 > KT || tail * sp * (128ll * 128 * 4) > ws_bytes)) break;
     if ((KT + sp - 1) / sp > kDeepMaxKt || (small >= 256 && KT > kDeepMaxKtRounds)) continue;
     const double t = deep_time(small, KT, sp, o);
     if (t < best) {
@@ -1398,12 +1403,14 @@ Plan plan_for(int64_t M, int64_t N, int KT, Output o, int64_t ws_bytes) {
 }
 
 // Bytes of partials the plan uses for an M x N x K product (0: no split),
-// whatever its output.
+// whatever its layout and output.
 int64_t split_bytes(int64_t M, int64_t N, int64_t K) {
   const int KT = static_cast<int>(K / BK);
   int64_t bytes = 0;
-  for (int o = 0; o < OUTPUTS; ++o) {
-    const Plan p = plan_for(M, N, KT, static_cast<Output>(o), kSplitCapBytes);
+  for (int v = 0; v < 2 * OUTPUTS; ++v) {
+    const int o = v >> 1;
+    const bool rows = v & 1;
+    const Plan p = plan_for(M, N, KT, rows, static_cast<Output>(o), kSplitCapBytes);
     int64_t b = 0;
     if (p.kind == DEEP && p.split > 1) {
       b = (((M + 127) / 128) * ((N + 127) / 128) % 256) * p.split * 128ll * 128 * 4;
@@ -1549,7 +1556,7 @@ int dispatch(GemmParams p, hipStream_t s) {
                        : EPI == EPI_SWIGLU_BWD ? OUT_SWIGLU_BWD
                        : OB                    ? OUT_B16
                                                : OUT_F32;
-  const Plan plan = plan_for(p.M, p.N, p.K / BK, o, p.ws ? p.ws_bytes : 0);
+  const Plan plan = plan_for(p.M, p.N, p.K / BK, AK, o, p.ws ? p.ws_bytes : 0);
   if (plan.kind == DEEP) return launch_deep<AK, BKM, EPI, OB>(p, plan.split, s);
   if (plan.kind == SMALL) return launch<128, 128, AK, BKM, EPI, OB>(p, s);
   return launch<256, 256, AK, BKM, EPI, OB>(p, s);

@@ -175,7 +175,7 @@ def test_4wave_k_split(layout, mnk):
 # tiles and splits.
 @pytest.mark.parametrize("layout", ["nt", "nn", "tn"])
 @pytest.mark.parametrize("mnk", [(264, 328, 64 * kt) for kt in (1, 2, 3, 4, 5, 9)]
-                         + [(128, 128, 4096), (584, 568, 4160), (5504, 760, 1280)])
+                         + [(128, 128, 6144), (584, 568, 6208), (5504, 760, 1280)])
 @pytest.mark.parametrize("kind", ["f32", "bf16 bias", "resid"])
 def test_deep(layout, mnk, kind):
     M, N, Kd = mnk
@@ -191,7 +191,7 @@ def test_deep(layout, mnk, kind):
         resid = torch.randn(M, N, generator=torch.Generator().manual_seed(183)).to(dev())
         ref = resid + ref
         bound = bound + ref.abs() * 2.0**-22
-    if Kd >= 4096:
+    if Kd >= 6144:
         assert K.gemm_workspace_bytes(M, N, Kd) > 0, "this shape is expected to split"
     out = torch.bfloat16 if bias is not None else torch.float32
     c = torch.full((M, N), 7.0, dtype=out, device=dev())
@@ -203,9 +203,24 @@ def test_deep(layout, mnk, kind):
     assert torch.equal(c, c8), "the deep and 8-wave kernels differ"
 
 
-@pytest.mark.parametrize("kd", [128, 2560])
+# Under 96 k-tiles a row's sums do not depend on how many rows come with it.
+@pytest.mark.parametrize("layout", ["nt", "nn"])
+@pytest.mark.parametrize("nk", [(256, 1536), (896, 4864)])
+def test_rows_keep_their_bits(layout, nk):
+    N, Kd = nk
+    print("case rows", layout, nk, flush=True, file=sys.stderr)
+    a, b, _, _ = _operands(layout, 2048, N, Kd, seed=200)
+    outs = []
+    for M in (128, 256, 520, 2048):
+        c = torch.empty(M, N, device=dev())
+        K.gemm(layout, a[:M], b, c, M=M, N=N, K=Kd)
+        outs.append(c)
+    assert all(torch.equal(c, outs[-1][:len(c)]) for c in outs)
+
+
+@pytest.mark.parametrize("kd", [128, 6144])
 def test_deep_swiglu(kd):
-    M, n = 392, 352  # 4 x 6 and 4 x 3 tiles with ragged edges; K = 2560 is cut
+    M, n = 392, 352  # 4 x 6 and 4 x 3 tiles with ragged edges; K = 6144 is cut
     print("case deep swiglu", kd, flush=True, file=sys.stderr)
     x, wd = _rand(M, kd, seed=190).to(dev()), _rand(kd, n, seed=193).to(dev())
     wgu = interleave_gate_up(_rand(n, kd, seed=191), _rand(n, kd, seed=192)).to(dev())
