@@ -334,6 +334,17 @@ int mr_gemm_swiglu(int64_t M, int64_t N, int64_t K, const void* X, int64_t ldx, 
                    size_t workspace_bytes, void* stream);
 
 /*
+ * The same with act written split for a split-precision product (order 0
+ * below): act_split [M, 3N] bf16 rows [hi | hi | lo], hi = bf16(act), lo =
+ * bf16(act - hi). act (hi alone, [M, N]) and gu come together, for a backward,
+ * or are both NULL. X and Wgu are themselves split operands there (K = 3 times
+ * the layer's). Alignment as above.
+ */
+int mr_gemm_swiglu_split(int64_t M, int64_t N, int64_t K, const void* X, int64_t ldx, const void* Wgu,
+                         int64_t ldw, void* act_split, int64_t ldsplit, void* act, int64_t ldact, void* gu,
+                         int64_t ldgu, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Input gradient of the down projection fused with the SwiGLU backward:
  * dact = dd Wd (dd [M, K] bf16, Wd [K, N] bf16 = down weight [hidden, inter]),
  * then from the saved gu (mr_gemm_swiglu's interleaved gate/up):

@@ -66,7 +66,9 @@ enum Epi : int {
   EPI_RESID = 1,   // C = resid[m, n] + acc (+ bias[n]), fp32
   EPI_SWIGLU = 2,  // act = silu(g) * u from row-interleaved gate/up weights
   EPI_SWIGLU_BWD = 3,  // dgu (interleaved) from dact = acc and the saved gate/up
+  EPI_SWIGLU_SPLIT = 4,  // SWIGLU with act written split, [hi | hi | lo] per row
 };
+constexpr bool is_swiglu(int epi) { return epi == EPI_SWIGLU || epi == EPI_SWIGLU_SPLIT; }
 
 struct GemmParams {
   int M, N, K;
@@ -82,6 +84,8 @@ struct GemmParams {
   int64_t ldr;
   uint16_t* gu;        // SWIGLU: gate/up copy, [M, 2 * n_out] bf16, interleaved like B
   int64_t ldgu;        // (SWIGLU_BWD reads the saved gate/up from gu and writes dgu to C)
+  uint16_t* act;       // SWIGLU_SPLIT: hi alone, [M, n_out] (with gu), or null; C holds the split rows
+  int64_t ldact;
   int grid_m, grid_n;
   // Tiles of this launch: logical tiles tile0 .. tile0 + n_tiles - 1 of the
   // grouped order. ksplit > 1: each tile's k steps are cut into ksplit runs
@@ -268,6 +272,9 @@ __device__ __forceinline__ void store16(T* p, T v) {
   else *p = v;
 }
 
+// What rounding x to bf16 leaves, exactly.
+__device__ __forceinline__ float bf16_rest(float x) { return x - bf16_to_f32(f32_to_bf16(x)); }
+
 // The epilogues of a wave's WM x WN share of a tile from its transposed
 // accumulators (see SWAP in the kernels), staged through the wave's REGION
 // bytes of LDS at `region` (free once the k loop has ended).
@@ -276,7 +283,7 @@ __device__ __forceinline__ void store_tile(const GemmParams& p, f32x16 (&acc)[TM
                                            int wn, int lane, uint8_t* region) {
   const int lrow = (lane >> 5) * 4;
   const int lcol = lane & 31;
-  if constexpr (EPI == EPI_SWIGLU) {
+  if constexpr (is_swiglu(EPI)) {
     // B rows interleave 32 gate rows and 32 up rows, and a wave's column
     // range starts on a multiple of 64: block j = 2q holds gate columns and
     // j = 2q + 1 the up columns of the same 32 act columns (accumulators are
@@ -287,6 +294,12 @@ __device__ __forceinline__ void store_tile(const GemmParams& p, f32x16 (&acc)[TM
     // and up copies as one 16-byte store each: whole cache lines instead of
     // 64-byte row pieces. (Computing act while staging made the compiler read
     // the accumulators out of the AGPRs ahead of the silu chains and spill.)
+    // SPLIT: act leaves as three pieces, bf16 hi twice and lo, a third of a row
+    // apart, and hi and the gate/up copies besides only where a backward will
+    // read them. (An fp32 gate/up product and a kernel that read it back moved
+    // 28 bytes an act column where this moves 6, a kernel of 157 us for 4096
+    // rows of 11008: a split-precision block forward of that size 1895 ->
+    // 1756 us, the same bits.)
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     typedef float f32x4 __attribute__((ext_vector_type(4)));
     typedef __attribute__((address_space(3))) uint8_t lds_u8;
@@ -304,6 +317,7 @@ __device__ __forceinline__ void store_tile(const GemmParams& p, f32x16 (&acc)[TM
     lds_u8* st = (lds_u8*)region;
     uint16_t* act = static_cast<uint16_t*>(p.C);
     const bool has_gu = p.gu != nullptr;
+    constexpr bool SPLIT = EPI == EPI_SWIGLU_SPLIT;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
 #pragma unroll
@@ -323,6 +337,7 @@ __device__ __forceinline__ void store_tile(const GemmParams& p, f32x16 (&acc)[TM
         // uniform bases of the slice; lane offsets stay 32-bit (ld < 2^22, 32 rows)
         uint16_t* const act_s = act + static_cast<int64_t>(row0) * p.ldc + col0 / 2;
         uint16_t* const gu_s = p.gu + static_cast<int64_t>(row0) * p.ldgu + col0;
+        uint16_t* const hi_s = SPLIT ? p.act + static_cast<int64_t>(row0) * p.ldact + col0 / 2 : nullptr;
         // (a slice wholly inside the outputs stores without per-lane guards,
         // as in the plain epilogue; N is a multiple of 32, so an act piece and
         // its gate and up pieces lie inside or past the edge together)
@@ -341,9 +356,18 @@ __device__ __forceinline__ void store_tile(const GemmParams& p, f32x16 (&acc)[TM
                 a[e] = silu(g0[e]) * u0[e];
                 a[e + 4] = silu(g1[e]) * u1[e];
               }
-              store16<false>(reinterpret_cast<u32x4*>(act_s + static_cast<uint32_t>(r * static_cast<int>(p.ldc) + ch * 8)),
-                      u32x4{pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3]), pack_bf16x2(a[4], a[5]),
-                            pack_bf16x2(a[6], a[7])});
+              const u32x4 hi = {pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3]), pack_bf16x2(a[4], a[5]),
+                                pack_bf16x2(a[6], a[7])};
+              uint16_t* const ao = act_s + static_cast<uint32_t>(r * static_cast<int>(p.ldc) + ch * 8);
+              store16<false>(reinterpret_cast<u32x4*>(ao), hi);
+              if constexpr (SPLIT) {
+                store16<false>(reinterpret_cast<u32x4*>(ao + p.n_out), hi);
+                store16<false>(reinterpret_cast<u32x4*>(ao + 2 * static_cast<int64_t>(p.n_out)),
+                               u32x4{pack_bf16x2(bf16_rest(a[0]), bf16_rest(a[1])), pack_bf16x2(bf16_rest(a[2]), bf16_rest(a[3])),
+                                     pack_bf16x2(bf16_rest(a[4]), bf16_rest(a[5])), pack_bf16x2(bf16_rest(a[6]), bf16_rest(a[7]))});
+                if constexpr (GU)
+                  store16<false>(reinterpret_cast<u32x4*>(hi_s + static_cast<uint32_t>(r * static_cast<int>(p.ldact) + ch * 8)), hi);
+              }
               if constexpr (GU) {
                 uint16_t* const o = gu_s + static_cast<uint32_t>(r * static_cast<int>(p.ldgu) + gc);
                 store16<false>(reinterpret_cast<u32x4*>(o), u32x4{pack_bf16x2(g0[0], g0[1]), pack_bf16x2(g0[2], g0[3]),
@@ -1218,7 +1242,7 @@ __global__ __launch_bounds__(64 * kWaves4) __attribute__((amdgpu_waves_per_eu(1,
 template <int BM, int BN, int EPI, bool OUT_BF16>
 __global__ __launch_bounds__(256) void gemm_reduce(GemmParams p) {
   typedef float f32x4 __attribute__((ext_vector_type(4)));
-  constexpr int NB = EPI == EPI_SWIGLU ? BN / 64 : BN / 32;  // blocks (or pairs) across a tile
+  constexpr int NB = is_swiglu(EPI) ? BN / 64 : BN / 32;  // blocks (or pairs) across a tile
   constexpr int PER_TILE = (BM / 32) * NB;
   const int t = static_cast<int>(blockIdx.x) / PER_TILE, rem = static_cast<int>(blockIdx.x) % PER_TILE;
   const int bi = rem / NB, bj = rem % NB;
@@ -1236,14 +1260,21 @@ __global__ __launch_bounds__(256) void gemm_reduce(GemmParams p) {
     return a;
   };
   auto pack4 = [](f32x4 v) { return make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])); };
-  if constexpr (EPI == EPI_SWIGLU) {
+  if constexpr (is_swiglu(EPI)) {
     const int col = (bn * BN) / 2 + bj * 32 + c * 4;  // act column; N and n_out are multiples of 32
     if (col >= p.n_out) return;
     const f32x4 g = sum4(2 * bj), u = sum4(2 * bj + 1);
     f32x4 a;
 #pragma unroll
     for (int k = 0; k < 4; ++k) a[k] = silu(g[k]) * u[k];
-    *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.C) + static_cast<int64_t>(row) * p.ldc + col) = pack4(a);
+    uint16_t* const ao = static_cast<uint16_t*>(p.C) + static_cast<int64_t>(row) * p.ldc + col;
+    *reinterpret_cast<uint2*>(ao) = pack4(a);
+    if constexpr (EPI == EPI_SWIGLU_SPLIT) {
+      *reinterpret_cast<uint2*>(ao + p.n_out) = pack4(a);
+      *reinterpret_cast<uint2*>(ao + 2 * static_cast<int64_t>(p.n_out)) =
+          pack4(f32x4{bf16_rest(a[0]), bf16_rest(a[1]), bf16_rest(a[2]), bf16_rest(a[3])});
+      if (p.gu) *reinterpret_cast<uint2*>(p.act + static_cast<int64_t>(row) * p.ldact + col) = pack4(a);
+    }
     if (p.gu) {
       uint16_t* o = p.gu + static_cast<int64_t>(row) * p.ldgu + bn * BN + bj * 64 + c * 4;
       *reinterpret_cast<uint2*>(o) = pack4(g);
@@ -1287,7 +1318,7 @@ __global__ __launch_bounds__(256) void gemm_reduce(GemmParams p) {
 
 template <int BM, int BN, int EPI, bool OUT_BF16>
 void launch_reduce(const GemmParams& p, hipStream_t s) {
-  constexpr int PER_TILE = (BM / 32) * (EPI == EPI_SWIGLU ? BN / 64 : BN / 32);
+  constexpr int PER_TILE = (BM / 32) * (is_swiglu(EPI) ? BN / 64 : BN / 32);
   hipLaunchKernelGGL((gemm_reduce<BM, BN, EPI, OUT_BF16>), dim3(static_cast<unsigned>(p.n_tiles) * PER_TILE), dim3(256),
                      0, s, p);
 }
@@ -1467,7 +1498,7 @@ int launch(GemmParams p, hipStream_t s) {
   constexpr int64_t wave = 256;
   const int64_t tail = tiles % wave, full = tiles - tail;
   const int split = BM == 256 && p.ws ? split_plan(tiles, KT, p.ws_bytes) : 1;
-  if constexpr (BM == 256 && EPI == EPI_STORE) {
+  if constexpr (BM == 256 && (EPI == EPI_STORE || EPI == EPI_SWIGLU_SPLIT)) {
     // A last wave at most half full runs as quarter tiles (two per CU)
     // instead of leaving half the CUs or more idle: measured 5-6 % faster on
     // the 7B block's q/k/v projection (4.5 waves) and its attention-output and
@@ -1554,6 +1585,7 @@ int dispatch(GemmParams p, hipStream_t s) {
   constexpr Output o = EPI == EPI_RESID        ? OUT_RESID
                        : EPI == EPI_SWIGLU     ? OUT_SWIGLU
                        : EPI == EPI_SWIGLU_BWD ? OUT_SWIGLU_BWD
+                       : EPI == EPI_SWIGLU_SPLIT ? OUT_F32  // the fp32 product's plan, so its bits
                        : OB                    ? OUT_B16
                                                : OUT_F32;
   const Plan plan = plan_for(p.M, p.N, p.K / BK, AK, o, p.ws ? p.ws_bytes : 0);
@@ -1613,6 +1645,52 @@ bool writes_overlap(const Region (&w)[NW], const Region (&r)[NR]) {
       if (w[b].p && overlap(w[a].p, w[a].n, w[b].p, w[b].n)) return true;
   }
   return false;
+}
+
+// mr_gemm_swiglu, or with `split` (rows of 3N) mr_gemm_swiglu_split, where
+// act is optional.
+int swiglu_product(const char* fn, int64_t M, int64_t N, int64_t K, const void* X, int64_t ldx, const void* Wgu,
+                   int64_t ldw, void* split, int64_t ldsplit, void* act, int64_t ldact, void* gu, int64_t ldgu,
+                   void* workspace, size_t workspace_bytes, void* stream) {
+  if (M <= 0 || N <= 0) return MR_OK;
+  if (!X || !Wgu || (!act && !split)) return fail(MR_EINVAL, "%s: null operand", fn);
+  if (M % 8 || N % 32 || K % BK || K <= 0)
+    return fail(MR_EINVAL, "%s: M %% 8, N %% 32 and K %% %d must be 0", fn, BK);
+  if (!ok16(X, ldx) || !ok16(Wgu, ldw) || (act && !ok16(act, ldact)) || (gu && !ok16(gu, ldgu)) ||
+      (split && !ok16(split, ldsplit)))
+    return fail(MR_EINVAL, "%s: operands and outputs must be 16-byte aligned with leading "
+                "dimensions multiples of 8", fn);
+  if (ldx < K || ldw < K || (act && ldact < N) || (gu && ldgu < 2 * N) || (split && ldsplit < 3 * N) || ldx > kMaxLd ||
+      ldw > kMaxLd || (act && ldact > kMaxLd) || (gu && ldgu > kMaxLd) || (split && ldsplit > kMaxLd))
+    return fail(MR_EINVAL, "%s: bad leading dimension", fn);
+  {
+    const Region w[4] = {{act, act ? span_bytes(M, ldact, N, 2) : 0}, {gu, gu ? span_bytes(M, ldgu, 2 * N, 2) : 0},
+                         {split, split ? span_bytes(M, ldsplit, 3 * N, 2) : 0},
+                         {workspace, static_cast<int64_t>(workspace_bytes)}};
+    const Region r[2] = {{X, span_bytes(M, ldx, K, 2)}, {Wgu, span_bytes(2 * N, ldw, K, 2)}};
+    if (writes_overlap(w, r))
+      return fail(MR_EINVAL, "%s: act, gu and the workspace must not overlap X, Wgu or each other", fn);
+  }
+  GemmParams p{};
+  p.M = static_cast<int>(M);
+  p.N = static_cast<int>(2 * N);
+  p.n_out = static_cast<int>(N);
+  p.K = static_cast<int>(K);
+  p.A = static_cast<const uint16_t*>(X);
+  p.lda = ldx;
+  p.B = static_cast<const uint16_t*>(Wgu);
+  p.ldb = ldw;
+  p.C = split ? split : act;
+  p.ldc = split ? ldsplit : ldact;
+  p.gu = static_cast<uint16_t*>(gu);
+  p.ldgu = ldgu;
+  if (!set_workspace(p, workspace, workspace_bytes))
+    return fail(MR_EINVAL, "%s: workspace must be 16-byte aligned", fn);
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  if (!split) return dispatch<true, true, EPI_SWIGLU, true>(p, s);
+  p.act = static_cast<uint16_t*>(act);
+  p.ldact = ldact;
+  return dispatch<true, true, EPI_SWIGLU_SPLIT, true>(p, s);
 }
 
 }  // namespace
@@ -1694,41 +1772,20 @@ int mr_gemm(int layout, int64_t M, int64_t N, int64_t K, const void* A, int64_t 
 int mr_gemm_swiglu(int64_t M, int64_t N, int64_t K, const void* X, int64_t ldx, const void* Wgu,
                    int64_t ldw, void* act, int64_t ldact, void* gu, int64_t ldgu, void* workspace,
                    size_t workspace_bytes, void* stream) {
-  using namespace mr;
-  clear_error();
+  mr::clear_error();
+  return mr::swiglu_product("mr_gemm_swiglu", M, N, K, X, ldx, Wgu, ldw, nullptr, 0, act, ldact, gu, ldgu, workspace,
+                            workspace_bytes, stream);
+}
+
+int mr_gemm_swiglu_split(int64_t M, int64_t N, int64_t K, const void* X, int64_t ldx, const void* Wgu,
+                         int64_t ldw, void* act_split, int64_t ldsplit, void* act, int64_t ldact, void* gu,
+                         int64_t ldgu, void* workspace, size_t workspace_bytes, void* stream) {
+  mr::clear_error();
   if (M <= 0 || N <= 0) return MR_OK;
-  if (!X || !Wgu || !act) return fail(MR_EINVAL, "mr_gemm_swiglu: null operand");
-  if (M % 8 || N % 32 || K % BK || K == 0)
-    return fail(MR_EINVAL, "mr_gemm_swiglu: M %% 8, N %% 32 and K %% %d must be 0", BK);
-  if (!ok16(X, ldx) || !ok16(Wgu, ldw) || !ok16(act, ldact) || (gu && !ok16(gu, ldgu)))
-    return fail(MR_EINVAL, "mr_gemm_swiglu: operands and outputs must be 16-byte aligned with leading "
-                "dimensions multiples of 8");
-  if (ldx < K || ldw < K || ldact < N || (gu && ldgu < 2 * N) || ldx > kMaxLd || ldw > kMaxLd ||
-      ldact > kMaxLd || (gu && ldgu > kMaxLd))
-    return fail(MR_EINVAL, "mr_gemm_swiglu: bad leading dimension");
-  {
-    const Region w[3] = {{act, span_bytes(M, ldact, N, 2)}, {gu, gu ? span_bytes(M, ldgu, 2 * N, 2) : 0},
-                         {workspace, static_cast<int64_t>(workspace_bytes)}};
-    const Region r[2] = {{X, span_bytes(M, ldx, K, 2)}, {Wgu, span_bytes(2 * N, ldw, K, 2)}};
-    if (writes_overlap(w, r))
-      return fail(MR_EINVAL, "mr_gemm_swiglu: act, gu and the workspace must not overlap X, Wgu or each other");
-  }
-  GemmParams p{};
-  p.M = static_cast<int>(M);
-  p.N = static_cast<int>(2 * N);
-  p.n_out = static_cast<int>(N);
-  p.K = static_cast<int>(K);
-  p.A = static_cast<const uint16_t*>(X);
-  p.lda = ldx;
-  p.B = static_cast<const uint16_t*>(Wgu);
-  p.ldb = ldw;
-  p.C = act;
-  p.ldc = ldact;
-  p.gu = static_cast<uint16_t*>(gu);
-  p.ldgu = ldgu;
-  if (!set_workspace(p, workspace, workspace_bytes))
-    return fail(MR_EINVAL, "mr_gemm_swiglu: workspace must be 16-byte aligned");
-  return dispatch<true, true, EPI_SWIGLU, true>(p, static_cast<hipStream_t>(stream));
+  if (!act_split) return mr::fail(MR_EINVAL, "mr_gemm_swiglu_split: null operand");
+  if (!act != !gu) return mr::fail(MR_EINVAL, "mr_gemm_swiglu_split: act and gu come together");
+  return mr::swiglu_product("mr_gemm_swiglu_split", M, N, K, X, ldx, Wgu, ldw, act_split, ldsplit, act, ldact, gu,
+                            ldgu, workspace, workspace_bytes, stream);
 }
 
 int mr_gemm_swiglu_bwd(int64_t M, int64_t N, int64_t K, const void* dd, int64_t ldd,

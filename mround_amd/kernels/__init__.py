@@ -83,6 +83,7 @@ _SIGNATURES = {
     "mr_gemm_f32_workspace_bytes": (ctypes.c_size_t, [_L, _L, _L]),
     "mr_gemm_f32_ws": (_I, [_I, _L, _L, _L, _P, _L, _P, _P, _L, _P, _L, _P, ctypes.c_size_t, _P]),
     "mr_gemm_swiglu": (_I, [_L, _L, _L, _P, _L, _P, _L, _P, _L, _P, _L, _P, ctypes.c_size_t, _P]),
+    "mr_gemm_swiglu_split": (_I, [_L, _L, _L, _P, _L, _P, _L, _P, _L, _P, _L, _P, _L, _P, ctypes.c_size_t, _P]),
     "mr_gemm_swiglu_bwd": (_I, [_L, _L, _L, _P, _L, _P, _L, _P, _L, _P, _L, _P, ctypes.c_size_t, _P]),
     "mr_rmsnorm_fwd": (_I, [_P, _P, _L, _L, _F, _P, _P, _P]),
     "mr_rmsnorm_bwd": (_I, [_P, _P, _P, _P, _P, _L, _L, _P, _P, _P]),
@@ -470,6 +471,21 @@ def gemm_swiglu(x, wgu, act, gu=None, *, workspace=None) -> None:
                               act.stride(0), _ptr(gu), gu.stride(0) if gu is not None else 0,
                               ws_ptr, ws_bytes, _stream(x))
     _check(rc, "mr_gemm_swiglu")
+
+
+def gemm_swiglu_split(x, wgu, act_split, act=None, gu=None, *, workspace=None) -> None:
+    """``mr_gemm_swiglu_split``: ``gemm_swiglu`` with act [hi | hi | lo] in
+    ``act_split`` [M, 3N], and hi alone and the gate/up values when given."""
+    M, K = x.shape
+    N = wgu.shape[0] // 2
+    if tuple(act_split.shape) != (M, 3 * N) or (act is not None and tuple(act.shape) != (M, N)) or (
+            gu is not None and tuple(gu.shape) != (M, 2 * N)):
+        raise KernelError("gemm_swiglu_split: act_split [M, 3N], act [M, N], gu [M, 2N]")
+    ws_ptr, ws_bytes = _ws_args(_gemm_ws(x.device, M, 2 * N, K, workspace))
+    rc = lib().mr_gemm_swiglu_split(M, N, K, _ptr(x), x.stride(0), _ptr(wgu), wgu.stride(0), _ptr(act_split),
+                                    act_split.stride(0), _ptr(act), act.stride(0) if act is not None else 0,
+                                    _ptr(gu), gu.stride(0) if gu is not None else 0, ws_ptr, ws_bytes, _stream(x))
+    _check(rc, "mr_gemm_swiglu_split")
 
 
 def gemm_swiglu_bwd(dd, wd, gu, dgu, *, workspace=None) -> None:

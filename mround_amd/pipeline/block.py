@@ -305,12 +305,12 @@ class BlockEngine:
         self.threshold = e(1, dt=f32)
         # split precision: fp32 W' and the split operands
         self.w32 = self.wqs = None
-        self.x1s = self.x2s = self.acts = self.gu32 = self.qkv32 = self.qkv_lo = self.attns = None
+        self.x1s = self.x2s = self.acts = self.qkv32 = self.qkv_lo = self.attns = None
         if self.split:
             self.w32 = {k: torch.empty(v.shape, dtype=f32, device=self.device) for k, v in self.wq.items()}
             self.wqs = {k: e(v.shape[0], 3 * v.shape[1]) for k, v in self.wq.items()}
             self.x1s, self.x2s = e(T, 3 * h), e(T, 3 * h)
-            self.acts, self.gu32 = e(T, 3 * mlp), e(T, 2 * mlp, dt=f32)
+            self.acts = e(T, 3 * mlp)
             self.qkv32, self.qkv_lo = e(T, shape.qkv_rows, dt=f32), e(T, shape.qkv_rows)
             self.attns = e(T, 3 * hq_d)
         self.cos_sin = rope_table(seq_len, shape.head_dim, shape.rope_theta, self.device, shape.rope_scaling)
@@ -337,7 +337,7 @@ class BlockEngine:
     PER_TOKEN = ("x1", "rstd1", "qkv", "attn", "h2", "x2", "rstd2", "act", "gu", "grad_out",
                  "grad_out16", "dgu", "dx2", "dh2", "dattn", "dqkv")
     PER_SEQUENCE = ("lse", "dsum")
-    SPLIT_PER_TOKEN = ("x1s", "x2s", "acts", "gu32", "qkv32", "qkv_lo", "attns")
+    SPLIT_PER_TOKEN = ("x1s", "x2s", "acts", "qkv32", "qkv_lo", "attns")
 
     def set_sequences(self, n: int) -> None:
         """Run the next passes over ``n`` sequences (at most the capacity the
@@ -450,7 +450,7 @@ class BlockEngine:
                 raise ArchitectureError("a saving forward needs its input kept: out must not be x")
             self.x_in = x
         if self.split:
-            self._forward_split(x, out)
+            self._forward_split(x, out, save)
             return
         K.rmsnorm_fwd(x, self.norm_in, s.norm_eps, self.x1, self.rstd1)
         self._run("gemm_qkv", lambda: K.gemm("nt", self.x1, self.wq["qkv"], self.qkv, M=T, N=s.qkv_rows,
@@ -468,7 +468,7 @@ class BlockEngine:
         self._run("gemm_down", lambda: K.gemm("nt", self.act, self.wq["down"], out, M=T, N=h, K=mlp,
                                               resid=self.h2, workspace=ws))
 
-    def _forward_split(self, x: torch.Tensor, out: torch.Tensor) -> None:
+    def _forward_split(self, x: torch.Tensor, out: torch.Tensor, save: bool) -> None:
         """``forward`` with the products in split precision (see the class);
         leaves the same saved activations (x1, x2 and act as their hi halves)."""
         s, T = self.shape, self.tokens
@@ -487,11 +487,9 @@ class BlockEngine:
         self._run("gemm_o", lambda: K.gemm("nt", self.attns, self.wqs["o"], self.h2, M=T, N=h, K=3 * hq_d,
                                            resid=x, workspace=ws))
         K.rmsnorm_fwd_split(self.h2, self.norm_post, s.norm_eps, self.x2s, self.x2, self.rstd2)
-
-        def gate_up():
-            K.gemm("nt", self.x2s, self.wqs["gu"], self.gu32, M=T, N=2 * mlp, K=3 * h, workspace=ws)
-            K.swiglu_split(self.gu32, self.acts, self.act, self.gu)
-        self._run("gemm_gate_up", gate_up)
+        self._run("gemm_gate_up", lambda: K.gemm_swiglu_split(
+            self.x2s, self.wqs["gu"], self.acts, self.act if save else None, self.gu if save else None,
+            workspace=ws))
         self._run("gemm_down", lambda: K.gemm("nt", self.acts, self.wqs["down"], out, M=T, N=h, K=3 * mlp,
                                               resid=self.h2, workspace=ws))
 

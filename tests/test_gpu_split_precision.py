@@ -436,3 +436,29 @@ def test_quantize_in_split_precision(tmp_path, bits, symmetry):
     assert rec["split_precision"] is True
     mem = rec["memory"]
     assert 0.85 * mem["peak"] <= mem["peak_allocated"] <= 1.05 * mem["peak"]
+
+
+# Ragged tiles, a tail cut along K (K 6144 and up) on the deep and the large
+# tiles, and whole rounds of large tiles.
+@pytest.mark.parametrize(("M", "N", "Kd"), [(8, 32, 64), (136, 96, 192), (264, 1536, 1728), (904, 352, 6144),
+                                            (512, 11008, 6144), (2048, 8576, 448)])
+@pytest.mark.parametrize("save", [True, False])
+def test_swiglu_split_epilogue(M, N, Kd, save):
+    """The fused form gives the bits of the fp32 gate/up product and ``swiglu_split``."""
+    _case("swiglu split epilogue", M, N, Kd, save)
+    gen = torch.Generator().manual_seed(N)
+    x = (torch.randn(M, Kd, generator=gen) * 0.3).to(dev(), torch.bfloat16)
+    w = (torch.randn(2 * N, Kd, generator=gen) * 0.1).to(dev(), torch.bfloat16)
+    act_s = torch.full((M, 3 * N), float("nan"), dtype=torch.bfloat16, device=dev())
+    act = torch.empty(M, N, dtype=torch.bfloat16, device=dev()) if save else None
+    gu = torch.empty(M, 2 * N, dtype=torch.bfloat16, device=dev()) if save else None
+    K.gemm_swiglu_split(x, w, act_s, act, gu)
+    gu32 = torch.empty(M, 2 * N, device=dev())
+    K.gemm("nt", x, w, gu32, M=M, N=2 * N, K=Kd)
+    want_s, want, want_gu = torch.empty_like(act_s), torch.empty(M, N, dtype=torch.bfloat16, device=dev()), \
+        torch.empty(M, 2 * N, dtype=torch.bfloat16, device=dev())
+    K.swiglu_split(gu32, want_s, want, want_gu)
+    assert torch.equal(act_s.view(torch.int16), want_s.view(torch.int16))
+    if save:
+        assert torch.equal(act.view(torch.int16), want.view(torch.int16))
+        assert torch.equal(gu.view(torch.int16), want_gu.view(torch.int16))
