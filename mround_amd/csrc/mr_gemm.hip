@@ -776,10 +776,10 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmParams p) {
     return;
   }
   {
-    constexpr int REGION = (BM + BN) * ROW_BYTES * 2 / kWaves;  // bytes of LDS per wave
-    static_assert(2 * REGION == BM * ROW_BYTES && 2 * REGION == BN * ROW_BYTES, "two waves per LDS array");
-    uint8_t* arr = wave < 2 ? As0 : wave < 4 ? As1 : wave < 6 ? Bs0 : Bs1;
-    store_tile<WM, WN, REGION, EPI, OUT_BF16>(p, acc, m0, n0, wm, wn, lane, arr + (wave & 1) * REGION);
+    // bytes of LDS per wave: two waves per array, or four per A array where A's are the larger
+    constexpr int REGION = BM == BN ? (BM + BN) * ROW_BYTES * 2 / kWaves : BM * ROW_BYTES / 4;
+    uint8_t* arr = BM == BN ? (wave < 2 ? As0 : wave < 4 ? As1 : wave < 6 ? Bs0 : Bs1) : wave < 4 ? As0 : As1;
+    store_tile<WM, WN, REGION, EPI, OUT_BF16>(p, acc, m0, n0, wm, wn, lane, arr + (wave & (BM == BN ? 1 : 3)) * REGION);
   }
 }
 
@@ -1018,7 +1018,7 @@ __global__ __launch_bounds__(64 * kWaves4) __attribute__((amdgpu_waves_per_eu(1,
   store_tile<WM, WN, STAGE, EPI, OUT_BF16>(p, acc, m0, n0, wm, wn, lane, region);
 }
 
-// ---- 4-wave kernel for 128 x 128 tiles on grids of at most one block per CU --
+// ---- deep-pipelined 4-wave kernel, 128 x 128 or 256 x 128 tiles, one block per CU --
 //
 // Where a launch has no more tiles than CUs (the small models' products, cut
 // along K or not), nothing but a block's own loads can hide the memory latency:
@@ -1035,18 +1035,27 @@ __global__ __launch_bounds__(64 * kWaves4) __attribute__((amdgpu_waves_per_eu(1,
 // Measured against the two-per-CU form: 576 x 576 x 4096 (25 tiles) 45 us, 26
 // here whole and 16 cut in 5; 4096 x 576 x 3072 34 -> 22; the residual products
 // 4096 x 576 x 1536 22 -> 16 and, on large tiles, 36; 2048 x 2048 x 2048 28 -> 20.
-template <bool A_KMAJOR, bool B_KMAJOR, int EPI, bool OUT_BF16>
+//
+// With BM = 256 (wide) a wave owns 128 x 64 and three stages of 48 KB take the
+// LDS: per product 3/4 of the operand reads and loads of the 128 x 128 form, for
+// grids that have too few 256 x 256 tiles and enough of these (operands in cache
+// and from memory, against the best other plan: 4096 x 1536 x 2048 30 -> 28 and
+// 40 -> 33 us; 1536 x 5120 x 4096 63 -> 55 and 69 -> 66; 9728 x 896 x 4096 75 ->
+// 70 and 84 -> 83; 8192 x 896 x 9728 131 -> 116 in cache).
+template <int BM, bool A_KMAJOR, bool B_KMAJOR, int EPI, bool OUT_BF16>
 __global__ __launch_bounds__(64 * kWaves4) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_deep_kernel(GemmParams p) {
-  constexpr int BM = 128, BN = 128, WM = 64, WN = 64, TM = 2, TN = 2;
-  constexpr int STAGE = BM * ROW_BYTES;
-  __shared__ __attribute__((aligned(1024))) uint8_t As0[STAGE];
-  __shared__ __attribute__((aligned(1024))) uint8_t As1[STAGE];
-  __shared__ __attribute__((aligned(1024))) uint8_t As2[STAGE];
-  __shared__ __attribute__((aligned(1024))) uint8_t As3[STAGE];
-  __shared__ __attribute__((aligned(1024))) uint8_t Bs0[STAGE];
-  __shared__ __attribute__((aligned(1024))) uint8_t Bs1[STAGE];
-  __shared__ __attribute__((aligned(1024))) uint8_t Bs2[STAGE];
-  __shared__ __attribute__((aligned(1024))) uint8_t Bs3[STAGE];
+  constexpr int BN = 128, WM = BM / 2, WN = 64, TM = WM / 32, TN = 2;
+  constexpr int STAGE_A = BM * ROW_BYTES, STAGE_B = BN * ROW_BYTES;
+  constexpr int NS = BM == 256 ? 3 : 4;      // stages
+  constexpr int LA = BM / 32, LB = BN / 32;  // a wave's loads of a k-tile
+  __shared__ __attribute__((aligned(1024))) uint8_t As0[STAGE_A];
+  __shared__ __attribute__((aligned(1024))) uint8_t As1[STAGE_A];
+  __shared__ __attribute__((aligned(1024))) uint8_t As2[STAGE_A];
+  __shared__ __attribute__((aligned(1024))) uint8_t As3[NS > 3 ? STAGE_A : 16];
+  __shared__ __attribute__((aligned(1024))) uint8_t Bs0[STAGE_B];
+  __shared__ __attribute__((aligned(1024))) uint8_t Bs1[STAGE_B];
+  __shared__ __attribute__((aligned(1024))) uint8_t Bs2[STAGE_B];
+  __shared__ __attribute__((aligned(1024))) uint8_t Bs3[NS > 3 ? STAGE_B : 16];
 
   // The first p.tile0 blocks take a whole tile each, the rest the (split, tile)
   // pairs of the tail, tiles fastest: each XCD a contiguous run of either, so
@@ -1111,8 +1120,7 @@ __global__ __launch_bounds__(64 * kWaves4) __attribute__((amdgpu_waves_per_eu(1,
   }
   typedef const __attribute__((address_space(3))) uint8_t* lds_ptr;
   bf16x8 af[2][TM], bfr[2][TN];
-  auto rd_tr = [](lds_ptr l, uint32_t reg, int kk) __attribute__((always_inline)) {
-    constexpr uint32_t R = MNMajorDirect<128>::ROWB;
+  auto rd_tr = [](lds_ptr l, uint32_t reg, int kk, uint32_t R) __attribute__((always_inline)) {  // R: bytes of a k-row
     const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t*)(l + reg + kk * 16 * R));
     const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16_t*)(l + reg + kk * 16 * R + 4 * R));
     return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
@@ -1121,12 +1129,12 @@ __global__ __launch_bounds__(64 * kWaves4) __attribute__((amdgpu_waves_per_eu(1,
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       if constexpr (A_KMAJOR) af[slot][i] = *(const lds_bf16x8_t*)(la + a_reg[kk] + i * 32 * ROW_BYTES);
-      else af[slot][i] = rd_tr(la, a_reg[i], kk);
+      else af[slot][i] = rd_tr(la, a_reg[i], kk, MNMajorDirect<BM>::ROWB);
     }
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       if constexpr (B_KMAJOR) bfr[slot][j] = *(const lds_bf16x8_t*)(lb + b_reg[kk] + j * 32 * ROW_BYTES);
-      else bfr[slot][j] = rd_tr(lb, b_reg[j], kk);
+      else bfr[slot][j] = rd_tr(lb, b_reg[j], kk, MNMajorDirect<BN>::ROWB);
     }
   };
   auto mm = [&](int slot) __attribute__((always_inline)) {
@@ -1137,46 +1145,63 @@ __global__ __launch_bounds__(64 * kWaves4) __attribute__((amdgpu_waves_per_eu(1,
         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bfr[slot][j], af[slot][i], acc[i][j], 0, 0, 0);
   };
   // The order of a k16 step: the next step's fragment reads and the loads
-  // between its 4 MFMAs.
+  // between its MFMAs.
   constexpr int NR = (A_KMAJOR ? TM : 2 * TM) + (B_KMAJOR ? TN : 2 * TN);
   auto order = [](bool loads) __attribute__((always_inline)) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      if (q < 2) __builtin_amdgcn_sched_group_barrier(0x100, NR / 2, 0);
+    for (int q = 0; q < TM * TN; ++q) {
+      if (q < TM * TN / 2) __builtin_amdgcn_sched_group_barrier(0x100, NR / (TM * TN / 2), 0);
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      if (loads) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
+      if (loads && q < (LA + LB) / 2) __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
   };
-  auto issue = [&](uint8_t* a, uint8_t* b, int i0, int i1) __attribute__((always_inline)) {
+  auto issue = [&](uint8_t* a, uint8_t* b, int h0, int h1) __attribute__((always_inline)) {  // halves h0 .. h1 - 1 of a k-tile
     const rsrc_t r_a = make_rsrc(at_a, 0x7fffffff), r_b = make_rsrc(at_b, 0x7fffffff);
 #pragma unroll
-    for (int i = i0; i < i1; ++i) {
-      ld_a.issue_one(r_a, i, a);
-      ld_b.issue_one(r_b, i, b);
-    }
+    for (int i = h0 * (LA / 2); i < h1 * (LA / 2); ++i) ld_a.issue_one(r_a, i, a);
+#pragma unroll
+    for (int i = h0 * (LB / 2); i < h1 * (LB / 2); ++i) ld_b.issue_one(r_b, i, b);
   };
-  const int phase = (4 - KT % 4) % 4;  // the stage k-tile 0 takes
+  const int phase = (NS - KT % NS) % NS;  // the stage k-tile 0 takes
   {
+    // The asm at the end differs between the phases, so that their first reads
+    // stay in place: merged behind the branches, their waits could not tell the
+    // stages apart (every load in flight was waited for), and with three phases
+    // the merged read lost its address in one of them.
     auto pro = [&](uint8_t* a0, uint8_t* b0, uint8_t* a1, uint8_t* b1, uint8_t* a2, uint8_t* b2, uint8_t* a3,
-                   uint8_t* b3) __attribute__((always_inline)) {
-      issue(a0, b0, 0, 4);
+                   uint8_t* b3, auto sc) __attribute__((always_inline)) {
+      issue(a0, b0, 0, 2);
       advance(1);
-      issue(a1, b1, 0, 4);
+      issue(a1, b1, 0, 2);
       advance(2);
-      issue(a2, b2, 0, 4);
-      advance(3);
-      issue(a3, b3, 0, 2);
-      asm volatile("s_waitcnt vmcnt(20)" ::: "memory");
+      if constexpr (NS == 4) {
+        issue(a2, b2, 0, 2);
+        advance(3);
+        issue(a3, b3, 0, 1);
+        asm volatile("s_waitcnt vmcnt(20)" ::: "memory");
+      } else {
+        issue(a2, b2, 0, 1);
+        asm volatile("s_waitcnt vmcnt(18)" ::: "memory");
+      }
       __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
       rd((lds_ptr)a0, (lds_ptr)b0, 0, 0);
+      asm volatile("; k-tile 0 in stage %0" ::"i"(decltype(sc)::value) : "memory");
     };
-    switch (phase) {
-      case 0: pro(As0, Bs0, As1, Bs1, As2, Bs2, As3, Bs3); break;
-      case 1: pro(As1, Bs1, As2, Bs2, As3, Bs3, As0, Bs0); break;
-      case 2: pro(As2, Bs2, As3, Bs3, As0, Bs0, As1, Bs1); break;
-      default: pro(As3, Bs3, As0, Bs0, As1, Bs1, As2, Bs2); break;
+    if constexpr (NS == 4) {
+      switch (phase) {
+        case 0: pro(As0, Bs0, As1, Bs1, As2, Bs2, As3, Bs3, std::integral_constant<int, 0>{}); break;
+        case 1: pro(As1, Bs1, As2, Bs2, As3, Bs3, As0, Bs0, std::integral_constant<int, 1>{}); break;
+        case 2: pro(As2, Bs2, As3, Bs3, As0, Bs0, As1, Bs1, std::integral_constant<int, 2>{}); break;
+        default: pro(As3, Bs3, As0, Bs0, As1, Bs1, As2, Bs2, std::integral_constant<int, 3>{}); break;
+      }
+    } else {
+      switch (phase) {
+        case 0: pro(As0, Bs0, As1, Bs1, As2, Bs2, As3, Bs3, std::integral_constant<int, 0>{}); break;
+        case 1: pro(As1, Bs1, As2, Bs2, As0, Bs0, As3, Bs3, std::integral_constant<int, 1>{}); break;
+        default: pro(As2, Bs2, As0, Bs0, As1, Bs1, As3, Bs3, std::integral_constant<int, 2>{}); break;
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -1185,42 +1210,45 @@ __global__ __launch_bounds__(64 * kWaves4) __attribute__((amdgpu_waves_per_eu(1,
     constexpr int S = decltype(sc)::value;
     uint8_t* la_ = S == 0 ? As0 : S == 1 ? As1 : S == 2 ? As2 : As3;
     uint8_t* lb_ = S == 0 ? Bs0 : S == 1 ? Bs1 : S == 2 ? Bs2 : Bs3;
-    uint8_t* na_ = S == 0 ? As1 : S == 1 ? As2 : S == 2 ? As3 : As0;  // k-tile u + 1
-    uint8_t* nb_ = S == 0 ? Bs1 : S == 1 ? Bs2 : S == 2 ? Bs3 : Bs0;
-    uint8_t* pa_ = S == 0 ? As3 : S == 1 ? As0 : S == 2 ? As1 : As2;  // k-tile u + 3
-    uint8_t* pb_ = S == 0 ? Bs3 : S == 1 ? Bs0 : S == 2 ? Bs1 : Bs2;
+    constexpr int N1 = (S + 1) % NS, P = (S + NS - 1) % NS;  // the stages of k-tiles u + 1 and u + NS - 1
+    uint8_t* na_ = N1 == 0 ? As0 : N1 == 1 ? As1 : N1 == 2 ? As2 : As3;
+    uint8_t* nb_ = N1 == 0 ? Bs0 : N1 == 1 ? Bs1 : N1 == 2 ? Bs2 : Bs3;
+    uint8_t* pa_ = P == 0 ? As0 : P == 1 ? As1 : P == 2 ? As2 : As3;
+    uint8_t* pb_ = P == 0 ? Bs0 : P == 1 ? Bs1 : P == 2 ? Bs2 : Bs3;
     const lds_ptr la = (lds_ptr)la_, lb = (lds_ptr)lb_;
     rd(la, lb, 1, 1);
-    issue(pa_, pb_, 2, 4);
+    issue(pa_, pb_, 1, 2);
     mm(0);
     order(true);
     rd(la, lb, 2, 0);
     mm(1);
     order(false);
     rd(la, lb, 3, 1);
-    advance(u + 4);
+    advance(u + NS);
     mm(0);
     order(false);
-    // Every read of this stage done, k-tile u + 1 landed (the 16 loads of
-    // k-tiles u + 2 and u + 3 may be in flight): a plain barrier, no fence.
-    asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)" ::: "memory");
+    // Every read of this stage done, k-tile u + 1 landed (the loads of the
+    // k-tiles after it may be in flight): a plain barrier, no fence.
+    if constexpr (NS == 4) asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(12) lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     rd((lds_ptr)na_, (lds_ptr)nb_, 0, 0);
-    issue(la_, lb_, 0, 2);
+    issue(la_, lb_, 0, 1);
     mm(1);
     order(true);
   };
   int u = 0;
   if (phase <= 0) tile(u++, std::integral_constant<int, 0>{});
   if (phase <= 1) tile(u++, std::integral_constant<int, 1>{});
-  if (phase <= 2) tile(u++, std::integral_constant<int, 2>{});
-  tile(u++, std::integral_constant<int, 3>{});
-  for (; u < KT; u += 4) {
+  if constexpr (NS == 4)
+    if (phase <= 2) tile(u++, std::integral_constant<int, 2>{});
+  tile(u++, std::integral_constant<int, NS - 1>{});
+  for (; u < KT; u += NS) {
     tile(u, std::integral_constant<int, 0>{});
     tile(u + 1, std::integral_constant<int, 1>{});
     tile(u + 2, std::integral_constant<int, 2>{});
-    tile(u + 3, std::integral_constant<int, 3>{});
+    if constexpr (NS == 4) tile(u + 3, std::integral_constant<int, 3>{});
   }
   // the repeated last loads land, every wave is past its reads: LDS is free
   __builtin_amdgcn_s_waitcnt(0);
@@ -1229,8 +1257,9 @@ __global__ __launch_bounds__(64 * kWaves4) __attribute__((amdgpu_waves_per_eu(1,
     store_partial<BM, BN>(p.ws + (static_cast<int64_t>(bid) * p.ksplit + split) * (BM * BN), acc, wm * TM, wn * TN, lane);
     return;
   }
-  uint8_t* region = wave == 0 ? As0 : wave == 1 ? As1 : wave == 2 ? As2 : As3;
-  store_tile<WM, WN, STAGE, EPI, OUT_BF16>(p, acc, m0, n0, wm, wn, lane, region);
+  constexpr int REGION = 128 * ROW_BYTES;
+  uint8_t* region = wave == 0 ? As0 : wave == 1 ? As1 : wave == 2 ? As2 : NS == 4 ? As3 : Bs0;
+  store_tile<WM, WN, REGION, EPI, OUT_BF16>(p, acc, m0, n0, wm, wn, lane, region);
 }
 
 // Sums the k-split partial tiles of a launch in split order and applies the
@@ -1349,60 +1378,68 @@ int split_plan(int64_t tiles, int KT, int64_t ws_bytes) {
   return split;
 }
 
-// How a product runs is whichever of three plans the times below expect to
-// take least. The constants are microseconds, fitted to 237 products (the
-// eleven of a block over geometries of hidden 512 .. 3584 and 256 .. 16384
-// tokens, and the vocabulary heads), each run by every plan: median error 4-6 %,
-// and the plan chosen is on average 1.3 % slower than the best of them. The
-// start and epilogue of a round of tiles depend on the kind of output.
+// How a product runs is whichever of four plans the times below expect to take
+// least. The constants are microseconds, fitted to 304 products (the twelve of
+// a block over geometries of hidden 576 .. 3584 and 256 .. 8192 tokens, and the
+// vocabulary heads), each run by every plan, with its operands in cache and, for
+// half of them, from memory: median error 4-8 %, and the plan chosen is on
+// average 0.8 % slower than the best of them. The start and epilogue of a round
+// of tiles depend on the kind of output.
 enum Output { OUT_B16, OUT_F32, OUT_RESID, OUT_SWIGLU, OUT_SWIGLU_BWD, OUTPUTS };
 
-// 128 x 128 tiles on the deep kernel, one block per CU: rounds of 256 tiles, the
-// tail past them cut along K into `split` blocks a tile, whose partials take a
-// round trip and a second kernel. A k-tile takes longer the more CUs work.
-double deep_time(int64_t tiles, int KT, int split, Output o) {
-  constexpr double start[OUTPUTS] = {2.4, 2.9, 3.9, 3.8, 5.0};
+// 128 x 128 or (wide) 256 x 128 tiles on the deep kernel, one block per CU:
+// rounds of 256, the tail past them cut along K into `split` blocks a tile, whose
+// partials take a round trip and a second kernel. A k-tile takes longer the more
+// CUs work.
+struct DeepTimes {
+  double launch, start[OUTPUTS], round, tail, busy, reduce, partial;
+};
+constexpr DeepTimes kDeepTimes = {0.9, {3.0, 4.0, 5.4, 4.9, 6.7}, 0.453, 0.305, 0.149, 1.2, 0.035};
+constexpr DeepTimes kWideTimes = {0.6, {4.3, 5.4, 7.5, 6.9, 11.0}, 0.838, 0.526, 0.266, 1.1, 0.051};
+double deep_time(const DeepTimes& c, int64_t tiles, int KT, int split, Output o) {
   const int64_t tail = tiles % 256, blocks = tail * split;
-  double t = 2.6 + static_cast<double>(tiles / 256) * (start[o] + 0.467 * KT);
-  if (tail) t += start[o] + (KT + split - 1) / split * (0.26 + 0.207 * static_cast<double>(blocks) / 256.0);
-  if (split > 1) t += 2.2 + 0.027 * static_cast<double>(blocks);
+  double t = c.launch + static_cast<double>(tiles / 256) * (c.start[o] + c.round * KT);
+  if (tail) t += c.start[o] + (KT + split - 1) / split * (c.tail + c.busy * static_cast<double>(blocks) / 256.0);
+  if (split > 1) t += c.reduce + c.partial * static_cast<double>(blocks);
   return t;
 }
 
 // The double-buffered 128 x 128 tiles, two blocks per CU: rounds of 512.
 double small_time(int64_t tiles, int KT, Output o) {
-  constexpr double start[OUTPUTS] = {1.1, 2.8, 3.2, 2.5, 5.9};
+  constexpr double start[OUTPUTS] = {2.0, 3.6, 4.8, 4.2, 7.7};
   const int64_t r = tiles % 512;
-  double t = 1.5 + static_cast<double>(tiles / 512) * (start[o] + 1.024 * KT);
-  if (r) t += start[o] + KT * (r <= 256 ? 0.601 : 0.749 + 0.275 * static_cast<double>(r - 256) / 256.0);
+  double t = static_cast<double>(tiles / 512) * (start[o] + 1.011 * KT);
+  if (r) t += start[o] + KT * (r <= 256 ? 0.642 : 0.832 + 0.195 * static_cast<double>(r - 256) / 256.0);
   return t;
 }
 
 // 256 x 256 tiles, one per CU: rounds of 256, the tail in `split` blocks a tile
 // or, up to half a round of plain stores, as quarter tiles (see launch).
 double big_time(int64_t tiles, int KT, int split, Output o) {
-  constexpr double start[OUTPUTS] = {8.2, 9.4, 12.2, 10.3, 18.8};
+  constexpr double start[OUTPUTS] = {7.5, 9.2, 12.1, 10.4, 18.9};
   const int64_t tail = tiles % 256, blocks = tail * split;
   double t = static_cast<double>(tiles / 256) * (start[o] + 1.481 * KT);
   if (tail && split == 1 && o <= OUT_F32 && tiles >= 256 && tail <= 128) {
-    t += start[o] + 0.66 * KT;
+    t += start[o] + 0.809 * KT;
   } else if (tail) {
     const double busy = blocks < 256 ? static_cast<double>(blocks) / 256.0 : 1.0;
-    t += static_cast<double>((blocks + 255) / 256) * (start[o] + (KT + split - 1) / split * (0.84 + 0.641 * busy));
+    t += static_cast<double>((blocks + 255) / 256) * (start[o] + (KT + split - 1) / split * (0.87 + 0.578 * busy));
   }
-  if (split > 1) t += 2.9 + 0.052 * static_cast<double>(blocks);
+  if (split > 1) t += 0.9 + 0.065 * static_cast<double>(blocks);
   return t;
 }
 
-enum Kind { BIG, SMALL, DEEP };
+enum Kind { BIG, SMALL, DEEP, WIDE };
 struct Plan {
   Kind kind;
-  int split;  // DEEP: blocks per tail tile
+  int split;  // DEEP, WIDE: blocks per tail tile
 };
 
 // In longer runs than these the deep kernel's k-tile slows beyond the fit (to
 // 0.6 us: 1024 x 3584 x 37888 took 359 us against 262 on split large tiles,
-// 9728 x 896 x 16384, two whole rounds, 353 against 290).
+// 9728 x 896 x 16384, two whole rounds, 353 against 290; on wide tiles
+// 4096 x 2048 x 11008, one round, 148 from cache and 177 from memory against 160
+// and 170 on large tiles).
 constexpr int kDeepMaxKt = 320, kDeepMaxKtRounds = 160;
 
 // The plan of an M x N x (64 KT) product with ws_bytes for partials. rows: M
@@ -1414,22 +1451,27 @@ constexpr int kDeepMaxKt = 320, kDeepMaxKtRounds = 160;
 Plan plan_for(int64_t M, int64_t N, int KT, bool rows, Output o, int64_t ws_bytes) {
   const int64_t big = ((M + 255) / 256) * ((N + 255) / 256);
   const int64_t small = ((M + 127) / 128) * ((N + 127) / 128);
+  const int64_t wide = ((M + 255) / 256) * ((N + 127) / 128);
   Plan p{BIG, 1};
   double best = big_time(big, KT, split_plan(big, KT, ws_bytes), o);
   if (small_time(small, KT, o) < best) {
     best = small_time(small, KT, o);
     p.kind = SMALL;
   }
-  const int64_t tail = small % 256;
-  for (int sp = 1; sp <= 16; ++sp) {
-    if (sp > 1 && (!tail || (rows && KT < kSplitMinKt) || tail * sp > 256 || sp * 2 > KT || tail * sp * (128ll * 128 * 4) > ws_bytes)) break;
-    if ((KT + sp - 1) / sp > kDeepMaxKt || (small >= 256 && KT > kDeepMaxKtRounds)) continue;
-    const double t = deep_time(small, KT, sp, o);
-    if (t < best) {
-      best = t;
-      p = Plan{DEEP, sp};
+  auto deep = [&](Kind kind, const DeepTimes& times, int64_t tiles, int64_t tile_bytes) {
+    const int64_t tail = tiles % 256;
+    for (int sp = 1; sp <= 16; ++sp) {
+      if (sp > 1 && (!tail || (rows && KT < kSplitMinKt) || tail * sp > 256 || sp * 2 > KT || tail * sp * tile_bytes > ws_bytes)) break;
+      if ((KT + sp - 1) / sp > kDeepMaxKt || (tiles >= 256 && KT > kDeepMaxKtRounds)) continue;
+      const double t = deep_time(times, tiles, KT, sp, o);
+      if (t < best) {
+        best = t;
+        p = Plan{kind, sp};
+      }
     }
-  }
+  };
+  deep(DEEP, kDeepTimes, small, 128ll * 128 * 4);
+  deep(WIDE, kWideTimes, wide, 256ll * 128 * 4);
   return p;
 }
 
@@ -1443,8 +1485,9 @@ int64_t split_bytes(int64_t M, int64_t N, int64_t K) {
     const bool rows = v & 1;
     const Plan p = plan_for(M, N, KT, rows, static_cast<Output>(o), kSplitCapBytes);
     int64_t b = 0;
-    if (p.kind == DEEP && p.split > 1) {
-      b = (((M + 127) / 128) * ((N + 127) / 128) % 256) * p.split * 128ll * 128 * 4;
+    if ((p.kind == DEEP || p.kind == WIDE) && p.split > 1) {
+      const int64_t bm = p.kind == WIDE ? 256 : 128;
+      b = (((M + bm - 1) / bm) * ((N + 127) / 128) % 256) * p.split * bm * 128 * 4;
     } else if (p.kind == BIG) {
       const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
       const int split = split_plan(tiles, KT, kSplitCapBytes);
@@ -1548,10 +1591,10 @@ int launch(GemmParams p, hipStream_t s) {
   return MR_OK;
 }
 
-// Small tiles on the deep kernel: whole rounds of 256, then the tail cut along K.
-template <bool AK, bool BKM, int EPI, bool OB>
+// BM x 128 tiles on the deep kernel: whole rounds of 256, then the tail cut along K.
+template <int BM, bool AK, bool BKM, int EPI, bool OB>
 int launch_deep(GemmParams p, int split, hipStream_t s) {
-  p.grid_m = (p.M + 127) / 128;
+  p.grid_m = (p.M + BM - 1) / BM;
   p.grid_n = (p.N + 127) / 128;
   const int64_t tiles = static_cast<int64_t>(p.grid_m) * p.grid_n;
   const int KT = p.K / BK;
@@ -1560,7 +1603,7 @@ int launch_deep(GemmParams p, int split, hipStream_t s) {
   p.kt_per = (KT + split - 1) / split;
   p.ksplit = (KT + p.kt_per - 1) / p.kt_per;  // no empty split
   if (use_4wave(KT)) {
-    hipLaunchKernelGGL((gemm_deep_kernel<AK, BKM, EPI, OB>), dim3(static_cast<unsigned>(p.tile0 + p.n_tiles * p.ksplit)),
+    hipLaunchKernelGGL((gemm_deep_kernel<BM, AK, BKM, EPI, OB>), dim3(static_cast<unsigned>(p.tile0 + p.n_tiles * p.ksplit)),
                        dim3(64 * kWaves4), 0, s, p);
   } else {  // the same tiles and splits on the 8-wave kernel
     GemmParams q = p;
@@ -1569,13 +1612,13 @@ int launch_deep(GemmParams p, int split, hipStream_t s) {
     q.ksplit = 1;
     q.kt_per = KT;
     if (q.n_tiles)
-      hipLaunchKernelGGL((gemm_kernel<128, 128, AK, BKM, EPI, OB>), dim3(static_cast<unsigned>(q.n_tiles)), dim3(kThreads),
+      hipLaunchKernelGGL((gemm_kernel<BM, 128, AK, BKM, EPI, OB>), dim3(static_cast<unsigned>(q.n_tiles)), dim3(kThreads),
                          0, s, q);
     if (p.n_tiles)
-      hipLaunchKernelGGL((gemm_kernel<128, 128, AK, BKM, EPI, OB>), dim3(static_cast<unsigned>(p.n_tiles * p.ksplit)),
+      hipLaunchKernelGGL((gemm_kernel<BM, 128, AK, BKM, EPI, OB>), dim3(static_cast<unsigned>(p.n_tiles * p.ksplit)),
                          dim3(kThreads), 0, s, p);
   }
-  if (p.n_tiles && p.ksplit > 1) launch_reduce<128, 128, EPI, OB>(p, s);
+  if (p.n_tiles && p.ksplit > 1) launch_reduce<BM, 128, EPI, OB>(p, s);
   MR_LAUNCH_CHECK("mr_gemm");
   return MR_OK;
 }
@@ -1589,7 +1632,8 @@ int dispatch(GemmParams p, hipStream_t s) {
                        : OB                    ? OUT_B16
                                                : OUT_F32;
   const Plan plan = plan_for(p.M, p.N, p.K / BK, AK, o, p.ws ? p.ws_bytes : 0);
-  if (plan.kind == DEEP) return launch_deep<AK, BKM, EPI, OB>(p, plan.split, s);
+  if (plan.kind == WIDE) return launch_deep<256, AK, BKM, EPI, OB>(p, plan.split, s);
+  if (plan.kind == DEEP) return launch_deep<128, AK, BKM, EPI, OB>(p, plan.split, s);
   if (plan.kind == SMALL) return launch<128, 128, AK, BKM, EPI, OB>(p, s);
   return launch<256, 256, AK, BKM, EPI, OB>(p, s);
 }

@@ -252,3 +252,38 @@ def test_deep_swiglu(kd):
     tol = torch.stack([(bd * u.abs() * 1.1).reshape(M, n // 32, 32), (bd * (g.abs() * sg)).reshape(M, n // 32, 32)], 2)
     got = dgu.float().reshape(M, n // 32, 2, 32)
     assert bool(torch.all((got - want).abs() <= tol + want.abs() * 2.0**-7 + 1e-6))
+
+
+# The deep kernel's 256 x 128 tiles (three LDS stages): every entry position into
+# the stage pattern (KT = 24, 25, 26), a longer K, ragged edges, and a grid past
+# one round (22 x 13 tiles) whose tail is cut along K.
+@pytest.mark.parametrize("layout", ["nt", "nn", "tn"])
+@pytest.mark.parametrize("mnk", [(2056, 3080, 64 * kt) for kt in (24, 25, 26, 64)] + [(5384, 1544, 6208)])
+@pytest.mark.parametrize("kind", ["f32", "bf16 bias", "resid"])
+def test_wide(layout, mnk, kind):
+    test_deep(layout, mnk, kind)
+
+
+@pytest.mark.parametrize("kt", [24, 25])
+def test_wide_swiglu(kt):
+    M, n, Kd = 2056, 1568, 64 * kt
+    print("case wide swiglu", (M, n, Kd), flush=True, file=sys.stderr)
+    x = _rand(M, Kd, seed=210).to(dev())
+    wgu = interleave_gate_up(_rand(n, Kd, seed=211), _rand(n, Kd, seed=212)).to(dev())
+    gu_ref, bound = _gpu_ref(x, wgu.t().contiguous())
+    dd, wd = _rand(M, Kd, seed=213).to(dev()), _rand(Kd, 3072, seed=214).to(dev())
+    saved = _rand(M, 6144, seed=215).to(dev())
+    outs = []
+    for wave8 in (False, True):
+        act, gu = (torch.empty(M, c, dtype=torch.bfloat16, device=dev()) for c in (n, 2 * n))
+        dgu = torch.empty(M, 6144, dtype=torch.bfloat16, device=dev())
+        if wave8:
+            with _EightWave():
+                K.gemm_swiglu(x, wgu, act, gu)
+                K.gemm_swiglu_bwd(dd, wd, saved, dgu)
+        else:
+            K.gemm_swiglu(x, wgu, act, gu)
+            K.gemm_swiglu_bwd(dd, wd, saved, dgu)
+        outs.append((act, gu, dgu))
+    assert all(torch.equal(a, b) for a, b in zip(*outs)), "the wide and 8-wave kernels differ"
+    assert bool(torch.all((outs[0][1].float() - gu_ref).abs() <= bound + gu_ref.abs() * 2.0**-8))
