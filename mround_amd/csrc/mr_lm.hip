@@ -158,6 +158,166 @@ __global__ __launch_bounds__(kCeBlock) void ce_rows(const uint16_t* logits, int6
   }
 }
 
+// The same with the row held in registers (rows of up to kHeldMax logits whose
+// starts are 16-byte aligned; V itself may be any number: one thread takes a last
+// partial piece element by element). What bounds ce_rows is memory, three passes
+// over rows that no cache keeps (2048 rows of 151936 logits are 622 MB); here a
+// row is read once. THREADS x N pieces of 8 logits cover the row, all of a
+// thread's loads in flight together: 1024 threads and 20 pieces fill a CU's
+// registers with one row of 163,840.
+// The largest logit is known before any exponential, so a logit costs one
+// multiply and v_exp_f32 in each of the two uses. That instruction gives zero
+// where the result is denormal: a row that reaches that far below its maximum
+// (or holds an infinity or a NaN) takes exp2f, on a second read.
+// Measured, 2048 rows: 151936 logits 368 -> 314 us (3.4 -> 4.0 TB/s of one read
+// and one write), 65536 143 -> 113, 16384 40 -> 29, 4000 18 -> 13, and 100001,
+// which ran the scalar kernel, 551 -> 213. (Whole rows of 1024 threads load, then
+// store: with two rows to a CU, up to 65536 logits, the two overlap.)
+constexpr int kHeldThreads = 1024, kHeldPieces = 20;
+constexpr int64_t kHeldMax = 8ll * kHeldThreads * kHeldPieces;
+
+template <int THREADS, int N>
+__global__ __launch_bounds__(THREADS, N <= 8 ? 8 : 4) void ce_rows_held(const uint16_t* logits, int64_t ld, int V,
+                                                        const int32_t* __restrict__ labels, float scale,
+                                                        float* __restrict__ row_loss, uint16_t* dlogits,
+                                                        int64_t ldd) {
+  constexpr int W = THREADS / 64;
+  constexpr uint32_t kNone = 0xff80ff80u;  // a pair of -inf: no part in the maximum or the sum
+  __shared__ float s_max[W], s_min[W], s_sum[W];
+  const int64_t row = blockIdx.x;
+  const uint16_t* x = logits + row * ld;
+  const uint4* x8 = reinterpret_cast<const uint4*>(x);
+  const int label = labels[row];
+  const int tid = threadIdx.x, n8 = V / 8, rest = V % 8;
+  float mx = -__builtin_inff(), mn = __builtin_inff();
+  uint4 r[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const int i = j * THREADS + tid;
+    r[j] = make_uint4(kNone, kNone, kNone, kNone);
+    if (i < n8) r[j] = x8[i];
+    else if (i == n8 && rest) {
+      uint32_t w[4] = {kNone, kNone, kNone, kNone};
+#pragma unroll
+      for (int k = 0; k < 7; ++k)
+        if (k < rest) {
+          const uint32_t v = x[n8 * 8 + k];
+          mn = fminf(mn, __uint_as_float(v << 16));
+          w[k >> 1] = (k & 1) ? (w[k >> 1] & 0xffffu) | (v << 16) : (w[k >> 1] & 0xffff0000u) | v;
+        }
+      r[j] = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+  }
+  // the label's logit, before the row may be overwritten in place
+  const bool ignored = label < 0;
+  const bool bad = label >= V;
+  float x_label = 0.0f;
+  if (tid == 0 && !ignored && !bad) x_label = bf16_to_f32(x[label]);
+  // (the values are unpacked anew in each pass, not kept: fresh hides that they are the same)
+  auto fresh = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) asm volatile("" : "+v"(r[j].x), "+v"(r[j].y), "+v"(r[j].z), "+v"(r[j].w));
+  };
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    float v[8];
+    unpack8(r[j], v);
+    float lo = v[0];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      mx = fmaxf(mx, v[k]);
+      lo = fminf(lo, v[k]);
+    }
+    if (j * THREADS + tid < n8) mn = fminf(mn, lo);
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+    mn = fminf(mn, __shfl_xor(mn, off, 64));
+  }
+  const int wave = tid >> 6;
+  if ((tid & 63) == 0) {
+    s_max[wave] = mx;
+    s_min[wave] = mn;
+  }
+  __syncthreads();
+  float m = s_max[0], least = s_min[0];
+#pragma unroll
+  for (int w = 1; w < W; ++w) {
+    m = fmaxf(m, s_max[w]);
+    least = fminf(least, s_min[w]);
+  }
+  // exp2's argument stays above -126 within 87 of the maximum
+  const bool normal = m - least < 87.0f;
+  float s = 0.0f;
+  fresh();
+  if (normal) {
+    float s1 = 0.0f;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      float v[8];
+      unpack8(r[j], v);
+#pragma unroll
+      for (int k = 0; k < 8; k += 2) {
+        s += __builtin_amdgcn_exp2f((v[k] - m) * kLog2e);
+        s1 += __builtin_amdgcn_exp2f((v[k + 1] - m) * kLog2e);
+      }
+    }
+    s += s1;
+  } else {
+    for (int i = tid; i < V; i += THREADS) s += exp2f((bf16_to_f32(x[i]) - m) * kLog2e);
+  }
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+  if ((tid & 63) == 0) s_sum[wave] = s;
+  __syncthreads();  // (and every read of the row is done)
+  s = s_sum[0];
+#pragma unroll
+  for (int w = 1; w < W; ++w) s += s_sum[w];
+  if (tid == 0) {
+    float l = 0.0f;
+    if (bad) {
+      l = __builtin_nanf("");
+    } else if (!ignored) {
+      l = m + log2f(s) * kLn2 - x_label;
+    }
+    row_loss[row] = l;
+  }
+  if (!dlogits) return;
+  uint16_t* d = dlogits + row * ldd;
+  const float g = ignored ? 0.0f : scale * (1.0f / s);
+  const int hot = ignored ? -1 : label;
+  if (!normal) {
+    for (int i = tid; i < V; i += THREADS) {
+      float p = exp2f((bf16_to_f32(x[i]) - m) * kLog2e) * g;
+      if (i == hot) p -= scale;
+      d[i] = f32_to_bf16(p);
+    }
+    return;
+  }
+  fresh();
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const int i = j * THREADS + tid;
+    if (i * 8 >= V) continue;
+    float v[8];
+    unpack8(r[j], v);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = __builtin_amdgcn_exp2f((v[k] - m) * kLog2e) * g;
+    if (hot >> 3 == i) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        if ((hot & 7) == k) v[k] -= scale;
+    }
+    if (i < n8) {
+      reinterpret_cast<uint4*>(d)[i] = make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]),
+                                                  pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
+    } else {
+#pragma unroll
+      for (int k = 0; k < 7; ++k)
+        if (k < rest) d[i * 8 + k] = f32_to_bf16(v[k]);
+    }
+  }
+}
+
 // loss = scale * sum of the row losses, in a fixed order (fp64 partials).
 __global__ __launch_bounds__(1024) void ce_finalize(const float* __restrict__ row_loss, int64_t T,
                                                     float scale, float* __restrict__ loss_out) {
@@ -227,9 +387,21 @@ int mr_cross_entropy(const void* logits, int64_t ld, int64_t T, int64_t V, const
   if (T > 0) {
     const uint16_t* x = static_cast<const uint16_t*>(logits);
     uint16_t* d = static_cast<uint16_t*>(dlogits);
-    const bool vec = V % 8 == 0 && ld % 8 == 0 && aligned16(x) &&
-                     (!d || (ldd % 8 == 0 && aligned16(d)));
-    if (vec)
+    const bool rows16 = ld % 8 == 0 && aligned16(x) && (!d || (ldd % 8 == 0 && aligned16(d)));
+    const bool vec = V % 8 == 0 && rows16;
+    const int64_t pieces = (V + 7) / 8;
+#define MR_CE(THREADS, N)                                                                                     \
+  hipLaunchKernelGGL((ce_rows_held<THREADS, N>), dim3(static_cast<unsigned>(T)), dim3(THREADS), 0, s, x, ld,  \
+                     static_cast<int>(V), labels, scale, row_loss, d, ldd)
+    // the fewest threads that hold the row in at most 8 pieces each, then more pieces
+    if (rows16 && pieces <= 256 * 4) MR_CE(256, 4);
+    else if (rows16 && pieces <= 256 * 8) MR_CE(256, 8);
+    else if (rows16 && pieces <= 512 * 8) MR_CE(512, 8);
+    else if (rows16 && pieces <= kHeldThreads * 8) MR_CE(kHeldThreads, 8);
+    else if (rows16 && pieces <= kHeldThreads * 14) MR_CE(kHeldThreads, 14);
+    else if (rows16 && V <= kHeldMax) MR_CE(kHeldThreads, kHeldPieces);
+#undef MR_CE
+    else if (vec)
       hipLaunchKernelGGL(ce_rows<true>, dim3(static_cast<unsigned>(T)), dim3(kCeBlock), 0, s, x, ld,
                          V, labels, scale, row_loss, d, ldd);
     else

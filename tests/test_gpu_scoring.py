@@ -86,6 +86,36 @@ def test_cross_entropy(T, V, inplace):
     assert torch.isnan(row[0]) and not torch.isnan(row[1:]).any()
 
 
+# Rows held in registers: the edges of each thread and piece count, vocabularies
+# that end inside a 16-byte piece, one past what is held, and rows that reach
+# below exp2's normal range (one by an infinity).
+@pytest.mark.parametrize("inplace", [False, True])
+@pytest.mark.parametrize("V", [5, 8191, 8193, 16385, 32769, 65536, 65537, 114689, 163833, 163841, 163848])
+def test_cross_entropy_held_rows(V, inplace):
+    _case("cross entropy held", V, inplace)
+    T, ld = 6, -(-V // 8) * 8 + 8
+    g = torch.Generator(device=dev()).manual_seed(V)
+    logits = torch.randn(T, ld, generator=g, device=dev()).mul_(3).to(torch.bfloat16)
+    logits[1, V - 1], logits[2, 0] = 20.0, -150.0
+    if V <= 163840:  # (the kernels past it make a NaN of one: a lane's running sum may meet it first)
+        logits[3, V // 2] = float("-inf")
+    pad = logits[:, V:].clone()
+    labels = torch.tensor([V - 1, V - 1, 1, 0, -1, V // 3], dtype=torch.int32, device=dev())
+    x = logits[:, :V].double()
+    ref_row = torch.logsumexp(x, 1) - x.gather(1, labels.clamp(min=0).long()[:, None])[:, 0]
+    ref_grad = torch.softmax(x, 1)
+    ref_grad[torch.arange(T, device=dev()), labels.clamp(min=0).long()] -= 1
+    ref_row[4], ref_grad[4] = 0, 0
+    row = torch.empty(T, device=dev())
+    dl = logits if inplace else torch.zeros_like(logits)
+    K.cross_entropy(logits, labels, V=V, scale=0.25, row_loss=row, dlogits=dl)
+    # sums of V float32 exponentials in at most 160-term runs; bf16 outputs
+    assert torch.allclose(row.double(), ref_row, rtol=1e-6, atol=1e-4)
+    err = (dl[:, :V].double() - 0.25 * ref_grad).abs()
+    assert bool((err <= 0.25 * ref_grad.abs() * 2.0**-8 + 1e-7 * 0.25).all()), float(err.max())
+    assert torch.equal(dl[:, V:], pad if inplace else torch.zeros_like(pad))
+
+
 def test_cross_entropy_rejects_bad_arguments():
     x = torch.zeros(4, 64, dtype=torch.bfloat16, device=dev())
     row = torch.empty(4, device=dev())
