@@ -1393,9 +1393,10 @@ enum Output { OUT_B16, OUT_F32, OUT_RESID, OUT_SWIGLU, OUT_SWIGLU_BWD, OUTPUTS }
 // CUs work.
 struct DeepTimes {
   double launch, start[OUTPUTS], round, tail, busy, reduce, partial;
+  int max_kt;  // longest run of k-tiles the fit holds for (see kDeepMaxKtRounds)
 };
-constexpr DeepTimes kDeepTimes = {0.9, {3.0, 4.0, 5.4, 4.9, 6.7}, 0.453, 0.305, 0.149, 1.2, 0.035};
-constexpr DeepTimes kWideTimes = {0.6, {4.3, 5.4, 7.5, 6.9, 11.0}, 0.838, 0.526, 0.266, 1.1, 0.051};
+constexpr DeepTimes kDeepTimes = {0.9, {3.0, 4.0, 5.4, 4.9, 6.7}, 0.453, 0.305, 0.149, 1.2, 0.035, 128};
+constexpr DeepTimes kWideTimes = {0.6, {4.3, 5.4, 7.5, 6.9, 11.0}, 0.838, 0.526, 0.266, 1.1, 0.051, 320};
 double deep_time(const DeepTimes& c, int64_t tiles, int KT, int split, Output o) {
   const int64_t tail = tiles % 256, blocks = tail * split;
   double t = c.launch + static_cast<double>(tiles / 256) * (c.start[o] + c.round * KT);
@@ -1435,12 +1436,13 @@ struct Plan {
   int split;  // DEEP, WIDE: blocks per tail tile
 };
 
-// In longer runs than these the deep kernel's k-tile slows beyond the fit (to
-// 0.6 us: 1024 x 3584 x 37888 took 359 us against 262 on split large tiles,
-// 9728 x 896 x 16384, two whole rounds, 353 against 290; on wide tiles
-// 4096 x 2048 x 11008, one round, 148 from cache and 177 from memory against 160
-// and 170 on large tiles).
-constexpr int kDeepMaxKt = 320, kDeepMaxKtRounds = 160;
+// In longer runs than max_kt, or than this in whole rounds, the k-tile slows
+// beyond the fit when operands come from memory (128 x 128 tiles to 0.6 us:
+// 4096 x 896 x 9728 64 us from cache and 91 from memory, 95 inside a 0.5B block
+// step, against 69 and 83 on wide tiles cut in two, the step 693 -> 688;
+// 9728 x 896 x 16384, two whole rounds, 353 against 290 on large tiles; on wide
+// tiles 4096 x 2048 x 11008, one round, 148 and 177 against 160 and 170).
+constexpr int kDeepMaxKtRounds = 160;
 
 // The plan of an M x N x (64 KT) product with ws_bytes for partials. rows: M
 // counts activation rows (NT, NN), not weight rows (TN). There a product of
@@ -1462,7 +1464,7 @@ Plan plan_for(int64_t M, int64_t N, int KT, bool rows, Output o, int64_t ws_byte
     const int64_t tail = tiles % 256;
     for (int sp = 1; sp <= 16; ++sp) {
       if (sp > 1 && (!tail || (rows && KT < kSplitMinKt) || tail * sp > 256 || sp * 2 > KT || tail * sp * tile_bytes > ws_bytes)) break;
-      if ((KT + sp - 1) / sp > kDeepMaxKt || (tiles >= 256 && KT > kDeepMaxKtRounds)) continue;
+      if ((KT + sp - 1) / sp > times.max_kt || (tiles >= 256 && KT > kDeepMaxKtRounds)) continue;
       const double t = deep_time(times, tiles, KT, sp, o);
       if (t < best) {
         best = t;
