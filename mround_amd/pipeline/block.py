@@ -468,9 +468,18 @@ class BlockEngine:
         self._run("gemm_down", lambda: K.gemm("nt", self.act, self.wq["down"], out, M=T, N=h, K=mlp,
                                               resid=self.h2, workspace=ws))
 
+    def linear_inputs(self) -> dict[str, torch.Tensor]:
+        """The bf16 inputs of the block's linears as the last forward, saving or
+        not, left them: ``x1`` (q/k/v), ``attn`` (o), ``x2`` (gate/up) and
+        ``act`` (down; in split precision the first hi segment of ``acts``, a
+        view whose rows are 3 inter apart)."""
+        act = self.acts[:, :self.shape.intermediate] if self.split else self.act
+        return {"x1": self.x1, "attn": self.attn, "x2": self.x2, "act": act}
+
     def _forward_split(self, x: torch.Tensor, out: torch.Tensor, save: bool) -> None:
         """``forward`` with the products in split precision (see the class);
-        leaves the same saved activations (x1, x2 and act as their hi halves)."""
+        leaves the same saved activations (x1, x2 and act as their hi halves),
+        act and gu only when saving: ``acts`` holds act's hi half either way."""
         s, T = self.shape, self.tokens
         h, hq_d, mlp = s.hidden, s.n_heads * s.head_dim, s.intermediate
         ws = self.gemm_ws

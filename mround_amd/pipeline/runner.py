@@ -422,12 +422,9 @@ class QuantizationRunner:
             for lo, hi in self._pieces(x):
                 eng.set_sequences((hi - lo) // seq)
                 eng.forward(x[lo:hi], scratch[lo:hi], save=False)
-                for t in (eng.x1, eng.attn, eng.x2, eng.act):
+                for name, t in eng.linear_inputs().items():
                     eng.zero_padding(t)  # token rows only
-                K.colsumsq(eng.x1, imp["x1"])
-                K.colsumsq(eng.attn, imp["attn"])
-                K.colsumsq(eng.x2, imp["x2"])
-                K.colsumsq(eng.act, imp["act"])
+                    K.colsumsq(t, imp[name])
         source = {"self_attn.q_proj": "x1", "self_attn.k_proj": "x1", "self_attn.v_proj": "x1",
                   "self_attn.o_proj": "attn", "mlp.gate_proj": "x2", "mlp.up_proj": "x2",
                   "mlp.down_proj": "act"}

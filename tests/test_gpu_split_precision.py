@@ -34,10 +34,11 @@ import torch
 
 from mround_amd import api
 from mround_amd import kernels as K
+from mround_amd.core.scale_search import search_scales
 from mround_amd.pipeline.block import LAYERS, BlockEngine, BlockShape, BlockWeights, placements, unplace
 from mround_amd.pipeline.checkpoint import write_random_checkpoint
-from mround_amd.pipeline.runner import DecoderBlock, QuantizationRunner
-from mround_amd.schemes import QuantScheme, Symmetry, TuningConfig
+from mround_amd.pipeline.runner import DecoderBlock, QuantizationRunner, _Layer
+from mround_amd.schemes import QuantScheme, ScaleInit, Symmetry, TuningConfig
 from oracle import block as OB
 from oracle import quantize as OQ
 from tests.helpers import dev
@@ -436,6 +437,52 @@ def test_quantize_in_split_precision(tmp_path, bits, symmetry):
     assert rec["split_precision"] is True
     mem = rec["memory"]
     assert 0.85 * mem["peak"] <= mem["peak_allocated"] <= 1.05 * mem["peak"]
+
+
+@pytest.mark.parametrize("split", [False, True])
+def test_search_weighs_what_the_forward_wrote(split):
+    """The searched scales of every layer are those of the float64 sums of
+    squares of its inputs, with nothing left over in the engine's buffers (all
+    filled with NaN ahead of the search), padded sequences and pieces included."""
+    _case("search inputs", split)
+    real, B = 100, 3
+    w = _weights(SMOLLM, seed=11)
+    scheme = QuantScheme(bits=2, group_size=64, symmetry=Symmetry.SYMMETRIC, scale_init=ScaleInit.SEARCHED)
+    tuning = TuningConfig(iters=1, batch_size=B, n_samples=2 * B, seq_len=real, micro_batches=2)
+    runner = QuantizationRunner(scheme, tuning, split_precision=split)
+    S = runner.rows
+    eng = runner.engine(SMOLLM, B * S, dev())
+    block = DecoderBlock(0, "b", SMOLLM, _dev(w))
+    eng.set_block(block.weights)
+    place = placements(SMOLLM)
+    layers = {n: _Layer(n, block.weights.linears[n], scheme, place[n]) for n in LAYERS}
+    gen = torch.Generator().manual_seed(12)
+    xs = [torch.randn(B * S, SMOLLM.hidden, generator=gen).to(dev()) for _ in range(2)]
+    for t in eng._full.values():
+        t.fill_(float("nan"))
+    assert runner._search_scales(eng, block, layers, xs)
+    # the same inputs from saving forwards, whose activations the backward reads
+    names = {"self_attn.q_proj": "x1", "self_attn.k_proj": "x1", "self_attn.v_proj": "x1",
+             "self_attn.o_proj": "attn", "mlp.gate_proj": "x2", "mlp.up_proj": "x2", "mlp.down_proj": "act"}
+    sums = {n: 0.0 for n in ("x1", "attn", "x2", "act")}
+    out = torch.empty_like(xs[0])
+    for x in xs:
+        for lo, hi in runner._pieces(x):
+            eng.set_sequences((hi - lo) // S)
+            eng.forward(x[lo:hi], out[lo:hi], save=True)
+            for n in sums:
+                t = getattr(eng, n)
+                sums[n] = sums[n] + (t.view(-1, S, t.shape[1])[:, :real].double() ** 2).sum((0, 1))
+    for n, layer in layers.items():
+        imp = sums[names[n]].float()
+        assert bool(torch.isfinite(imp).all())
+        want = search_scales(layer.weight, scheme, importance=imp)
+        got = layer.init_scale.reshape(-1, 1)
+        # fp32 sums in another order (2^-16 of the importance at most) may tip a
+        # near-tie between neighbouring candidates, in few of a layer's groups
+        differ = float((got != want).double().mean())
+        print(f"  {n}: {differ:.2e} of the scales differ", file=sys.stderr)
+        assert bool(torch.isfinite(got).all()) and differ <= 2e-3, n
 
 
 # Ragged tiles, a tail cut along K (K 6144 and up) on the deep and the large
