@@ -14,14 +14,14 @@
 // h + m + l is x. Of the nine plane products the six down to 2^-16 of the
 // largest are formed (each exact in the MFMA): h h into one accumulator and
 // h m + m h + h l + m m + l h into a second, added once at the end. The three
-// left out are at most 2^-25 of a product together, under the rounding of a
-// float32 product; the sum itself rounds once per 16 k instead of once per
-// 2 k. Measured against float64 over K = 64 .. 6000: 0.15-0.4 of the fp32 MFMA
+// left out are at most 2^-24 of a product together, as much as a float32
+// product's own rounding; the sum itself rounds once per 16 k instead of once
+// per 2 k. Measured against float64 over K = 64 .. 6000: 0.15-0.4 of the fp32 MFMA
 // form's error (normwise 5e-8 .. 4e-7 against 1.4e-7 .. 1.4e-6).
 //
 // The split is exact while l's last bit stays in bfloat16's range and h does
-// not overflow. A block that met a nonzero |x| below 2^-100, or whose sums are
-// not all finite (an infinity or a NaN among its operands makes them so, as a
+// not overflow. A block that met a nonzero |x| below 2^-100 (tested on x, not on
+// h: below 2^-133 h itself rounds to zero), or whose sums are not all finite (an infinity or a NaN among its operands makes them so, as a
 // value that rounds to infinity does), forms its tile again with the fp32
 // MFMA, so infinities, NaNs and denormals come out as float32 arithmetic has
 // them.
@@ -54,7 +54,6 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int TM = 128, TN = 128, TK = 32;
 constexpr int kThreads = 256;
@@ -63,9 +62,9 @@ constexpr int PAD = 4;                   // LDS row padding of the fp32 form (fl
 constexpr int PLANE = TM * TK * 2;       // bytes of one plane of one operand tile
 constexpr int kStage = 6 * PLANE;        // both operands
 static_assert(TM == TN && 2 * kStage >= 2 * TK * (TM + PAD) * 4, "the fp32 form stages in the same LDS");
-// Smallest admissible (h << 1) - 2 of a nonzero h plane, 2^-100 (zeros wrap to
+// Smallest admissible (bits << 1) - 2 of a nonzero value, 2^-100 (zeros wrap to
 // the top).
-constexpr uint16_t kKeyLo = ((127 - 100) << 8) - 2;
+constexpr uint32_t kKeyLo = ((127u - 100u) << 24) - 2;
 
 struct Operand {
   const float* x;
@@ -155,7 +154,7 @@ struct Share {
     }
   }
   // The share's three planes; `key` collects the smallest magnitude key.
-  __device__ __forceinline__ void split(Planes& p, u16x2& key) const {
+  __device__ __forceinline__ void split(Planes& p, uint32_t& key) const {
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -166,8 +165,7 @@ struct Share {
           b = b - y[j][2 * q + 1];
         }
         const uint32_t h = pack_bf16x2(a, b);
-        const u16x2 h2 = __builtin_bit_cast(u16x2, h);
-        key = __builtin_elementwise_min(key, static_cast<u16x2>(h2 * u16x2{2, 2} - u16x2{2, 2}));
+        key = min(key, min((__float_as_uint(a) << 1) - 2, (__float_as_uint(b) << 1) - 2));
         const float a1 = a - __uint_as_float(h << 16), b1 = b - __uint_as_float(h & 0xffff0000u);
         const uint32_t m = pack_bf16x2(a1, b1);
         p.v[j][0][q] = h;
@@ -254,7 +252,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_f32_kernel(Gemm32 p) {
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = low[i][j] = f32x16{};
-  u16x2 key = {0xffff, 0xffff};
+  uint32_t key = 0xffffffffu;
 
   Share<A_KMAJOR, PAIRS, false> sa[2];
   Share<B_KMAJOR, PAIRS, MINUS> sb[2];
@@ -363,7 +361,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_f32_kernel(Gemm32 p) {
       mul(fr[0]);
     }
   }
-  bool bad = min(key.x, key.y) < kKeyLo;
+  bool bad = key < kKeyLo;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int m = m0 + wm * 64 + i * 32 + l32;

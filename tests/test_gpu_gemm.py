@@ -401,6 +401,35 @@ def test_gemm_f32_split(layout, mnk, pad):
     assert torch.all((c.double().cpu() - want).abs() <= bound)
 
 
+# A lone value under 2^-133, whose bfloat16 planes are all zero, against operands
+# large enough for the product to be an ordinary number: in a whole k tile, in
+# the rest of K past the last one, as an operand's own value and as B - B2.
+@pytest.mark.parametrize("layout", ["nt", "nn", "tn"])
+@pytest.mark.parametrize("where", ["a", "b", "b - b2"])
+@pytest.mark.parametrize("exponent", [-133, -134, -140, -149])
+def test_gemm_f32_smallest(layout, where, exponent):
+    M, N, Kd = 140, 136, 609
+    print("case gemm f32 smallest", layout, where, exponent, flush=True, file=sys.stderr)
+    g = torch.Generator().manual_seed(6)
+    small, large = torch.zeros(M if where == "a" else N, Kd), torch.randn(N if where == "a" else M, Kd, generator=g)
+    for r, k in ((133, 40), (2, 608)):  # (one value of a block's, in either part of K)
+        small[r, k] = 2.0**exponent
+    large *= 1e30
+    a, b = (small, large) if where == "a" else (large, small)
+    b2 = None
+    if where == "b - b2":
+        b2 = torch.randn(N, Kd, generator=g)
+        b2[small != 0] = -(2.0**exponent)
+        b = torch.where(small != 0, torch.zeros(()), b2)
+    want = a.double() @ small.double().T if where != "a" else small.double() @ b.double().T
+    A = (a if layout != "tn" else a.T.contiguous()).to(dev())
+    B, B2 = ((t if layout == "nt" else t.T.contiguous()).to(dev()) if t is not None else None for t in (b, b2))
+    c = torch.empty(M, N, device=dev())
+    K.gemm_f32(layout, A, B, c, M=M, N=N, K=Kd, b_minus=B2)
+    # (one nonzero product an output, exact but for the denormal's own bits: 2^-23)
+    assert torch.all((c.double().cpu() - want).abs() <= want.abs() * 2.0**-23 + 2.0**-149)
+
+
 # Values outside the three-plane split's range: infinities, NaNs, magnitudes at
 # the top of float32 and far below its normal range come out as float32 has them.
 @pytest.mark.parametrize("layout", ["nt", "tn"])
