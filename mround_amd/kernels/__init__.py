@@ -413,19 +413,13 @@ def gemm_workspace_bytes(M: int, N: int, K: int) -> int:
 
 
 def _gemm_ws(device: torch.device, M: int, N: int, K: int, workspace):
-    """The caller's workspace, or the binding's own per-device one grown to the
-    plan's size (the library allocates nothing)."""
+    """The caller's workspace, or a tensor of the call's own of the plan's size
+    (the library allocates nothing): the allocator ties it to the current
+    stream, so calls on several streams share no partials."""
     if workspace is not None:
         return workspace
     nbytes = gemm_workspace_bytes(M, N, K)
-    if nbytes == 0:
-        return None
-    key = (device.index or 0, "gemm")
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
-        _workspaces[key] = ws
-    return ws
+    return torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None
 
 
 def _ws_args(ws):
@@ -435,7 +429,7 @@ def _ws_args(ws):
 def gemm(layout: str, a, b, c, *, M, N, K, bias=None, resid=None, workspace=None) -> None:
     """``mr_gemm``: C = op(A) op(B) (+ bias) (+ resid); leading dims from strides.
     ``workspace``: the k-split partials (a device tensor of at least
-    ``gemm_workspace_bytes(M, N, K)`` bytes); None uses the binding's own."""
+    ``gemm_workspace_bytes(M, N, K)`` bytes); None allocates them for the call."""
     ws_ptr, ws_bytes = _ws_args(_gemm_ws(a.device, M, N, K, workspace))
     rc = lib().mr_gemm(GEMM_LAYOUT[layout], M, N, K, _rows_ptr(a), a.stride(0), _rows_ptr(b), b.stride(0),
                        _rows_ptr(c), dtype_code(c.dtype), c.stride(0), _ptr(_f32(bias, "bias")),

@@ -167,6 +167,21 @@ def test_gemm_workspace_unsplit_shapes(lib, M, N, K):
     assert lib.mr_gemm_workspace_bytes(M, N, K) == 0
 
 
+def test_gemm_calls_share_no_workspace(lib):
+    # a weight gradient of short K, cut along K: without a workspace each call
+    # has partials of its own, so that calls on two streams do not meet in them
+    import torch
+
+    from mround_amd import kernels as K
+
+    cpu, mnk = torch.device("cpu"), (576, 576, 4096)
+    assert K.gemm_workspace_bytes(*mnk) > 0
+    one, two = (K._gemm_ws(cpu, *mnk, None) for _ in range(2))
+    assert one.numel() == two.numel() == K.gemm_workspace_bytes(*mnk)
+    assert one.data_ptr() != two.data_ptr()
+    assert K._gemm_ws(cpu, *mnk, one) is one  # the caller's own is used as it is
+
+
 def test_attention_workspace_follows_the_head_split(lib):
     T = 8 * 2048
     # 7B: 4 kv heads x 8 x 16 key blocks = 512 blocks, no split

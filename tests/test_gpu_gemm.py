@@ -337,6 +337,28 @@ def test_gemm_residual_every_layout(layout, mnk, inplace):
 
 
 # ------------------------------------------------------------------ fp32 GEMM --
+# Weight gradients whose tiles are cut along K, without a workspace, on two
+# streams at once: each gives the bits it gives alone.
+def test_gemm_on_two_streams():
+    M, N, Kd = 576, 576, 4096
+    print("case gemm two streams", flush=True, file=sys.stderr)
+    assert K.gemm_workspace_bytes(M, N, Kd) > 0  # the k-split path
+    ops = [(_rand(Kd, M, seed=s).to(dev()), _rand(Kd, N, seed=s + 1).to(dev())) for s in (301, 303)]
+    want = []
+    for a, b in ops:
+        want.append(torch.empty(M, N, device=dev()))
+        K.gemm("tn", a, b, want[-1], M=M, N=N, K=Kd)
+    outs = [[torch.empty(M, N, device=dev()) for _ in range(50)] for _ in ops]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in ops]
+    for i in range(50):
+        for s, (a, b), out in zip(streams, ops, outs):
+            with torch.cuda.stream(s):
+                K.gemm("tn", a, b, out[i], M=M, N=N, K=Kd)
+    torch.cuda.synchronize()
+    assert all(torch.equal(c, w) for out, w in zip(outs, want) for c in out)
+
+
 # mr_gemm_f32, the single-layer loop's products: fp32 products and
 # accumulation, any sizes, B - B2 formed as the operand is loaded. Bound: the
 # float64 product of the same fp32 operands within (K + 4) 2^-23 of the sum of
