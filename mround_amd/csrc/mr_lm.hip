@@ -33,12 +33,15 @@ __device__ __forceinline__ MaxSum merge(MaxSum a, MaxSum b) {
   return {m, a.s * exp2f((a.m - m) * kLog2e) + b.s * exp2f((b.m - m) * kLog2e)};
 }
 
-// Adds n values held in x[] to the running pair with one rescale.
+// Adds n values held in x[] to the running pair with one rescale. (Values that
+// are all -inf sum to zero, an empty pair; taken from themselves they would be
+// NaNs, as they are where one of them is a NaN.)
 template <int N>
 __device__ __forceinline__ MaxSum absorb(MaxSum acc, const float (&x)[N]) {
   float mx = x[0];
 #pragma unroll
   for (int k = 1; k < N; ++k) mx = fmaxf(mx, x[k]);
+  if (mx == -__builtin_inff()) mx = 0.0f;
   float s = 0.0f;
 #pragma unroll
   for (int k = 0; k < N; ++k) s += exp2f((x[k] - mx) * kLog2e);

@@ -97,8 +97,7 @@ def test_cross_entropy_held_rows(V, inplace):
     g = torch.Generator(device=dev()).manual_seed(V)
     logits = torch.randn(T, ld, generator=g, device=dev()).mul_(3).to(torch.bfloat16)
     logits[1, V - 1], logits[2, 0] = 20.0, -150.0
-    if V <= 163840:  # (the kernels past it make a NaN of one: a lane's running sum may meet it first)
-        logits[3, V // 2] = float("-inf")
+    logits[3, V // 2] = float("-inf")
     pad = logits[:, V:].clone()
     labels = torch.tensor([V - 1, V - 1, 1, 0, -1, V // 3], dtype=torch.int32, device=dev())
     x = logits[:, :V].double()
@@ -114,6 +113,38 @@ def test_cross_entropy_held_rows(V, inplace):
     err = (dl[:, :V].double() - 0.25 * ref_grad).abs()
     assert bool((err <= 0.25 * ref_grad.abs() * 2.0**-8 + 1e-7 * 0.25).all()), float(err.max())
     assert torch.equal(dl[:, V:], pad if inplace else torch.zeros_like(pad))
+
+
+# Infinite logits, wherever a lane's share of the row meets them (its first
+# values, all of them, most of the vocabulary masked): -inf takes no part in the
+# sum and no gradient; a NaN, also among -inf, and +inf make the row's loss NaN.
+# Aligned rows, rows that start off 16 bytes, and rows past what registers hold.
+@pytest.mark.parametrize("V,ld", [(250, 256), (4096, 4099), (65536, 65537), (163841, 163848), (163848, 163848)])
+def test_cross_entropy_infinities(V, ld):
+    _case("cross entropy infinities", V, ld)
+    inf = float("inf")
+    g = torch.Generator(device=dev()).manual_seed(V)
+    logits = torch.randn(8, ld, generator=g, device=dev()).mul_(3).to(torch.bfloat16)
+    logits[0, 0] = -inf
+    logits[1, :V - 3] = -inf
+    logits[2, 1:] = -inf
+    logits[3, ::2] = -inf
+    logits[4, :64] = -inf
+    logits[5, 100:200], logits[5, 133] = -inf, float("nan")
+    logits[6, 70] = inf
+    labels = torch.tensor([V - 1, V - 1, 0, 3, 101, 7, 70, V // 2], dtype=torch.int32, device=dev())
+    x = logits[:, :V].double()
+    ref_row = torch.logsumexp(x, 1) - x.gather(1, labels.long()[:, None])[:, 0]
+    ref_grad = torch.softmax(x, 1)
+    ref_grad[torch.arange(8, device=dev()), labels.long()] -= 1
+    nan = torch.zeros(8, dtype=torch.bool, device=dev())
+    nan[5:7] = True
+    row, dl = torch.empty(8, device=dev()), torch.zeros_like(logits)
+    K.cross_entropy(logits, labels, V=V, scale=0.25, row_loss=row, dlogits=dl)
+    assert torch.equal(row.isnan(), nan)
+    assert torch.allclose(row.double()[~nan], ref_row[~nan], rtol=1e-6, atol=1e-4)
+    err = (dl[~nan, :V].double() - 0.25 * ref_grad[~nan]).abs()
+    assert bool((err <= 0.25 * ref_grad[~nan].abs() * 2.0**-8 + 1e-7 * 0.25).all()), float(err.max())
 
 
 def test_cross_entropy_rejects_bad_arguments():
