@@ -170,12 +170,14 @@ __global__ __launch_bounds__(kCeBlock) void ce_rows(const uint16_t* logits, int6
 // registers with one row of 163,840.
 // The largest logit is known before any exponential, so a logit costs one
 // multiply and v_exp_f32 in each of the two uses. That instruction gives zero
-// where the result is denormal: a row that reaches that far below its maximum
-// (or holds an infinity or a NaN) takes exp2f, on a second read.
+// where the result is denormal: the gradient of a row that reaches that far
+// below its maximum (or holds an infinity) takes exp2f.
 // Measured, 2048 rows: 151936 logits 368 -> 314 us (3.4 -> 4.0 TB/s of one read
 // and one write), 65536 143 -> 113, 16384 40 -> 29, 4000 18 -> 13, and 100001,
 // which ran the scalar kernel, 551 -> 213. (Whole rows of 1024 threads load, then
-// store: with two rows to a CU, up to 65536 logits, the two overlap.)
+// store: with two rows to a CU, up to 65536 logits, the two overlap.) With a -inf in
+// every row 151936 logits take 371, 65536 118 and 100001 247 us; second reads of such
+// rows an element at a time took 970, 261 and 637.
 constexpr int kHeldThreads = 1024, kHeldPieces = 20;
 constexpr int64_t kHeldMax = 8ll * kHeldThreads * kHeldPieces;
 
@@ -250,11 +252,18 @@ __global__ __launch_bounds__(THREADS, N <= 8 ? 8 : 4) void ce_rows_held(const ui
     least = fminf(least, s_min[w]);
   }
   // exp2's argument stays above -126 within 87 of the maximum
-  const bool normal = m - least < 87.0f;
-  float s = 0.0f;
+  const bool normal = __builtin_expect(m - least < 87.0f, 1);
+  // A piece for the rows outside: one at a time, its arithmetic apart from what
+  // ordinary rows do (shared with theirs, the pieces spilled).
+  auto apart = [&](int j, float (&v)[8]) __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+    uint4 p = r[j];
+    asm volatile("; below the normal range" : "+v"(p.x), "+v"(p.y), "+v"(p.z), "+v"(p.w));
+    unpack8(p, v);
+  };
+  float s = 0.0f, s1 = 0.0f;
   fresh();
   if (normal) {
-    float s1 = 0.0f;
 #pragma unroll
     for (int j = 0; j < N; ++j) {
       float v[8];
@@ -265,10 +274,19 @@ __global__ __launch_bounds__(THREADS, N <= 8 ? 8 : 4) void ce_rows_held(const ui
         s1 += __builtin_amdgcn_exp2f((v[k + 1] - m) * kLog2e);
       }
     }
-    s += s1;
-  } else {
-    for (int i = tid; i < V; i += THREADS) s += exp2f((bf16_to_f32(x[i]) - m) * kLog2e);
+  } else {  // (terms made zero are under 2^-126 of a sum of at least 1)
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      float v[8];
+      apart(j, v);
+#pragma unroll
+      for (int k = 0; k < 8; k += 2) {
+        s += __builtin_amdgcn_exp2f((v[k] - m) * kLog2e);
+        s1 += __builtin_amdgcn_exp2f((v[k + 1] - m) * kLog2e);
+      }
+    }
   }
+  s += s1;
   for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
   if ((tid & 63) == 0) s_sum[wave] = s;
   __syncthreads();  // (and every read of the row is done)
@@ -288,23 +306,7 @@ __global__ __launch_bounds__(THREADS, N <= 8 ? 8 : 4) void ce_rows_held(const ui
   uint16_t* d = dlogits + row * ldd;
   const float g = ignored ? 0.0f : scale * (1.0f / s);
   const int hot = ignored ? -1 : label;
-  if (!normal) {
-    for (int i = tid; i < V; i += THREADS) {
-      float p = exp2f((bf16_to_f32(x[i]) - m) * kLog2e) * g;
-      if (i == hot) p -= scale;
-      d[i] = f32_to_bf16(p);
-    }
-    return;
-  }
-  fresh();
-#pragma unroll
-  for (int j = 0; j < N; ++j) {
-    const int i = j * THREADS + tid;
-    if (i * 8 >= V) continue;
-    float v[8];
-    unpack8(r[j], v);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = __builtin_amdgcn_exp2f((v[k] - m) * kLog2e) * g;
+  auto store = [&](int i, float (&v)[8]) __attribute__((always_inline)) {
     if (hot >> 3 == i) {
 #pragma unroll
       for (int k = 0; k < 8; ++k)
@@ -318,6 +320,30 @@ __global__ __launch_bounds__(THREADS, N <= 8 ? 8 : 4) void ce_rows_held(const ui
       for (int k = 0; k < 7; ++k)
         if (k < rest) d[i * 8 + k] = f32_to_bf16(v[k]);
     }
+  };
+  if (!normal) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const int i = j * THREADS + tid;
+      if (i * 8 >= V) continue;
+      float v[8];
+      apart(j, v);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = exp2f((v[k] - m) * kLog2e) * g;
+      store(i, v);
+    }
+    return;
+  }
+  fresh();
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const int i = j * THREADS + tid;
+    if (i * 8 >= V) continue;
+    float v[8];
+    unpack8(r[j], v);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = __builtin_amdgcn_exp2f((v[k] - m) * kLog2e) * g;
+    store(i, v);
   }
 }
 

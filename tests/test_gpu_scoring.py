@@ -12,6 +12,7 @@ results (embedding rows, DeltaLoss terms) are exact.
 from __future__ import annotations
 
 import json
+import math
 import sys
 
 import numpy as np
@@ -145,6 +146,25 @@ def test_cross_entropy_infinities(V, ld):
     assert torch.allclose(row.double()[~nan], ref_row[~nan], rtol=1e-6, atol=1e-4)
     err = (dl[~nan, :V].double() - 0.25 * ref_grad[~nan]).abs()
     assert bool((err <= 0.25 * ref_grad[~nan].abs() * 2.0**-8 + 1e-7 * 0.25).all()), float(err.max())
+
+
+# A row 90 below its maximum: the exponentials are denormal, and so are the
+# gradients, which keep their value (half a bf16 denormal's step of 2^-133, and
+# float32's rounding of exp's argument at 130 and of its denormal result).
+@pytest.mark.parametrize("V", [250, 4096, 16384, 65536, 100001, 151936, 163848])
+def test_cross_entropy_denormal_gradients(V):
+    _case("cross entropy denormal", V)
+    ld = -(-V // 8) * 8
+    logits = torch.full((3, ld), -30.0, dtype=torch.bfloat16, device=dev())
+    logits[0, 0] = logits[1, V // 2] = logits[2, V - 1] = 60.0
+    labels = torch.tensor([0, V // 2, V - 1], dtype=torch.int32, device=dev())
+    row, dl = torch.empty(3, device=dev()), torch.zeros_like(logits)
+    K.cross_entropy(logits, labels, V=V, scale=1.0, row_loss=row, dlogits=dl)
+    want = math.exp(-90.0)
+    got = dl[:, :V].double()
+    got[torch.arange(3), labels.long()] = want  # (the label's own: a sum that rounds to 1, less 1)
+    assert bool(((got - want).abs() <= 2.0**-134 + 2.0**-149 + want * 2.0**-15).all())
+    assert bool((row.abs() <= 1e-6).all())
 
 
 def test_cross_entropy_rejects_bad_arguments():
