@@ -157,8 +157,12 @@ __device__ __forceinline__ void store8(void* p, int64_t i, const float (&x)[8]) 
       if constexpr (DT == MR_BF16) {
         words[k] = pack_bf16x2(x[2 * k], x[2 * k + 1]);
       } else {
-        words[k] = static_cast<uint32_t>(f32_to_f16(x[2 * k])) |
-                   (static_cast<uint32_t>(f32_to_f16(x[2 * k + 1])) << 16);
+        // the float32 values themselves: folded into the product that made
+        // them (v_fma_mixlo_f16) the narrowing rounds only once and a zero
+        // loses its sign
+        float lo = x[2 * k], hi = x[2 * k + 1];
+        asm("" : "+v"(lo), "+v"(hi));
+        words[k] = static_cast<uint32_t>(f32_to_f16(lo)) | (static_cast<uint32_t>(f32_to_f16(hi)) << 16);
       }
     }
     st16_stream(static_cast<uint16_t*>(p) + i, make_uint4(words[0], words[1], words[2], words[3]));

@@ -316,3 +316,22 @@ def test_long_groups_and_float16(mode, shape, wdtype):
         assert torch.equal(placed[2:rows + 2], nxt) and bool((placed[:2] == 7).all()) and bool((placed[rows + 2:] == 7).all())
         seen.append(outs[2])
     assert torch.equal(*seen)
+
+
+# A float16 W' is the float32 W' narrowed, bit for bit: two roundings, and the
+# sign of a zero (vector kernels, groups in registers, and a wave per group).
+@pytest.mark.parametrize("mode", ["asym", "sym", "searched"])
+@pytest.mark.parametrize("shape", [(576, 1536, 64), (512, 256, 8), (512, 1024, 512), (64, 4864, -1), (64, 600, 40)])
+@pytest.mark.parametrize("wdtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_float16_output_is_the_narrowed_float32(mode, shape, wdtype):
+    rows, cols, gs = shape
+    _note("float16 output", mode, shape, wdtype)
+    w = weight(rows, cols, seed=7, dtype=wdtype).to(dev())
+    v, a, b = (t.to(dev()) for t in params(rows, cols, gs, seed=8, coef_jitter=0.5))
+    init = _init_scale(rows, cols, gs).to(dev()) if mode == "searched" else None
+    scheme = _scheme(mode, 4, gs)
+    for p in ({"v": v, "alpha": a, "beta": b}, None):
+        wide, narrow = (QZ.fake_quantize(w, p, scheme, init_scale=init, out_dtype=dt)
+                        for dt in (torch.float32, torch.float16))
+        want = to_np(wide).astype(np.float16)
+        assert np.array_equal(to_np(narrow).view(np.int16), want.view(np.int16))
