@@ -804,13 +804,15 @@ __global__ __launch_bounds__(kBlock) void fq_bwd_generic(
 //
 // Per-channel groups (one scale a row) and other groups of 256 weights and
 // more that are not 8 * 2^k: T threads (a wave, four or sixteen) own a group, each
-// up to kRowChunks runs of 8 consecutive weights, so that W, v and the gradient
-// are read once, in 16-byte loads, before the extremes are known, and the
-// backward's sums need no second read. HBM-bound. The wave-per-group form
-// read each operand two or three times, 2 or 4 bytes a lane: measured on a
-// float16 4864 x 896 weight with one group a row, forward 21 and fused step 23
-// us, 8 and 16 here (3.5 and 4.7 TB/s past the launch). (Two runs a thread for
-// the shorter groups, half the registers, measured the same.)
+// up to C runs of 8 consecutive weights (1, 2 or kRowChunks: no more registers
+// than the group needs), so that W, v and the gradient are read once, in 16-byte
+// loads, before the extremes are known, and the backward's sums need no second
+// read. HBM-bound. The wave-per-group form read each operand two or three times,
+// 2 or 4 bytes a lane: measured on a float16 4864 x 896 weight with one group a
+// row, forward 21 and fused step 23 us, 8 and 16 here (3.5 and 4.7 TB/s past the
+// launch). On 8 M bfloat16 weights, forward and step in us, wave per group, four
+// runs a thread whatever the group, and C runs: groups of 384 28 + 32, 15.5 + 33,
+// 14.6 + 29; of 8200 136 + 155, 21 + 61, 16 + 39.
 constexpr int kRowChunks = 4;
 
 __device__ __forceinline__ void load8_any(const void* p, int dt, int64_t e, float (&x)[8]) {
@@ -861,12 +863,12 @@ __device__ __forceinline__ int64_t row_group(int& t) {
   return blockIdx.x;
 }
 
-template <int MODE, int T>
-__device__ __forceinline__ void row_extremes(const float (&x)[kRowChunks][8], int nc, int t, float* sm, float& mx, float& mn) {
+template <int MODE, int T, int C>
+__device__ __forceinline__ void row_extremes(const float (&x)[C][8], int nc, int t, float* sm, float& mx, float& mn) {
   mx = mn = 0.0f;  // (the extremes are taken with zero)
   if constexpr (MODE != MR_SYM_SEARCHED) {
 #pragma unroll
-    for (int k = 0; k < kRowChunks; ++k) {
+    for (int k = 0; k < C; ++k) {
       if (t + k * T >= nc) continue;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
@@ -879,7 +881,7 @@ __device__ __forceinline__ void row_extremes(const float (&x)[kRowChunks][8], in
   }
 }
 
-template <int MODE, bool HAS_V, int T>
+template <int MODE, bool HAS_V, int T, int C>
 __global__ __launch_bounds__(T == 64 ? kBlock : T) void fq_fwd_row(
     const void* __restrict__ w, int wt, const float* __restrict__ v, const float* __restrict__ alpha,
     const float* __restrict__ beta, const float* __restrict__ init_scale, void* __restrict__ wq, int ot,
@@ -890,9 +892,9 @@ __global__ __launch_bounds__(T == 64 ? kBlock : T) void fq_fwd_row(
   const int64_t grp = row_group<T>(t);
   if (grp >= n_groups) return;  // (whole waves, and only where no barrier follows)
   const int nc = gs / 8;
-  float x[kRowChunks][8], vv[kRowChunks][8];
+  float x[C][8], vv[C][8];
 #pragma unroll
-  for (int k = 0; k < kRowChunks; ++k) {
+  for (int k = 0; k < C; ++k) {
     const int c = t + k * T;
     if (c >= nc) continue;
     load8_any(w, wt, grp * gs + c * 8, x[k]);
@@ -909,7 +911,7 @@ __global__ __launch_bounds__(T == 64 ? kBlock : T) void fq_fwd_row(
   const Group p = group_params<MODE>(mx, mn, a, b, base, maxq, inv_maxq, eps);
   const int64_t out = wq ? map.row(grp / ng) * cols + (grp % ng) * gs : 0;
 #pragma unroll
-  for (int k = 0; k < kRowChunks; ++k) {
+  for (int k = 0; k < C; ++k) {
     const int c = t + k * T;
     if (c >= nc) continue;
     float lmx = mx, lmn = mn;
@@ -945,7 +947,7 @@ __global__ __launch_bounds__(T == 64 ? kBlock : T) void fq_fwd_row(
   }
 }
 
-template <int MODE, bool UPDATE, int T>
+template <int MODE, bool UPDATE, int T, int C>
 __global__ __launch_bounds__(T == 64 ? kBlock : T) void fq_bwd_row(
     const void* __restrict__ w, int wt, float* __restrict__ v, float* __restrict__ alpha, float* __restrict__ beta,
     const float* __restrict__ init_scale, const void* __restrict__ g, int gt, int64_t n_groups, int64_t cols, int gs,
@@ -958,9 +960,9 @@ __global__ __launch_bounds__(T == 64 ? kBlock : T) void fq_bwd_row(
   if (grp >= n_groups) return;
   const int nc = gs / 8;
   const int64_t placed = map.row(grp / ng) * cols + (grp % ng) * gs;
-  float x[kRowChunks][8], vv[kRowChunks][8], gg[kRowChunks][8];
+  float x[C][8], vv[C][8], gg[C][8];
 #pragma unroll
-  for (int k = 0; k < kRowChunks; ++k) {
+  for (int k = 0; k < C; ++k) {
     const int c = t + k * T;
     if (c >= nc) continue;
     load8_any(w, wt, grp * gs + c * 8, x[k]);
@@ -987,7 +989,7 @@ __global__ __launch_bounds__(T == 64 ? kBlock : T) void fq_bwd_row(
   };
   float sum_s = 0.0f, sum_d = 0.0f;
 #pragma unroll
-  for (int k = 0; k < kRowChunks; ++k) {
+  for (int k = 0; k < C; ++k) {
     const int c = t + k * T;
     if (c >= nc) continue;
     float lmx, lmn, tq[8];
@@ -1026,7 +1028,7 @@ __global__ __launch_bounds__(T == 64 ? kBlock : T) void fq_bwd_row(
     if (st.wq) {
       const Group p2 = group_params<MODE>(mx, mn, na, nb, base, maxq, inv_maxq, eps);
 #pragma unroll
-      for (int k = 0; k < kRowChunks; ++k) {
+      for (int k = 0; k < C; ++k) {
         const int c = t + k * T;
         if (c >= nc) continue;
         float lmx, lmn, tq[8], q[8];
@@ -1096,6 +1098,29 @@ int row_threads(int gs) {
   return gs <= 64 * 8 * kRowChunks ? 64 : gs <= 256 * 8 * kRowChunks ? 256 : 1024;
 }
 
+// Runs of 8 that a thread of T holds: 1, 2 or 4.
+int row_chunks(int gs, int T) {
+  const int c = (gs / 8 + T - 1) / T;
+  return c > 2 ? 4 : c;
+}
+
+// Whether the backward of row groups takes the row kernels. On grids of 8
+// waves a SIMD and more (4 searched), the wave-per-group kernel rereads groups of up to 2048
+// weights (a wave each) from the caches, and is the faster where much of the wave's last run of 8 is idle, and in the
+// searched mode (no pass for the extremes) for all but long 16-bit groups. Step
+// on 8 M weights, wave per group and row kernel in us: groups of 320 float32
+// asymmetric 30.0 and 32.1, bfloat16 34.5 and 32.5, of 352 31.2 and 31.0, 34.7
+// and 31.0, of 520 30.6 and 32.2 (9.4 and 7.2 where 2016 of them are all), of
+// 1032 31.3 and 31.4; searched, groups of 480
+// 25.0 and 24.7, 27.5 and 25.7, of 640 22.1 and 27.4, 24.3 and 27.7, of 768 23.5
+// and 25.3, 26.8 and 24.7, of 2048 float32 24.0 and 27.4, of 2560 28.0 and 25.4.
+bool row_backward(const Shape& sh, int mode, int wt) {
+  const int runs = sh.gs / 8;
+  if (runs > 256 || sh.n_groups < (mode == MR_SYM_SEARCHED ? 4096 : 8192)) return true;
+  const bool full = runs * 100 >= 65 * 64 * row_chunks(sh.gs, 64);  // of the slots that T = 64 gives it
+  return mode == MR_SYM_SEARCHED ? wt != MR_F32 && runs >= 96 && full : runs > 128 || full;
+}
+
 template <int MODE, bool HAS_V>
 int launch_fwd(const Shape& sh, const void* w, int wt, const float* v, const float* alpha,
                const float* beta, const float* init_scale, void* wq, int ot, uint8_t* codes,
@@ -1135,13 +1160,18 @@ int launch_fwd(const Shape& sh, const void* w, int wt, const float* v, const flo
     const int T = row_threads(sh.gs);
     const int64_t blocks = T == 64 ? (sh.n_groups + 3) / 4 : sh.n_groups;
     if (blocks > 0x7fffffff) return fail(MR_EINVAL, "mr_fq_forward: tensor too large");
-#define MR_FWD_ROW(T_)                                                                                         \
-  hipLaunchKernelGGL((fq_fwd_row<MODE, HAS_V, T_>), dim3(static_cast<unsigned>(blocks)), dim3(T_ == 64 ? kBlock : T_), \
+#define MR_FWD_ROW(T_, C_)                                                                                     \
+  hipLaunchKernelGGL((fq_fwd_row<MODE, HAS_V, T_, C_>), dim3(static_cast<unsigned>(blocks)), dim3(T_ == 64 ? kBlock : T_), \
                      0, stream, w, wt, v, alpha, beta, init_scale, wq, ot, codes, scale_out, zp_out, sh.n_groups,  \
                      sh.cols, sh.gs, sh.ng, sh.maxq, sh.inv_maxq, sh.qmin, sh.qmax, eps, map)
-    if (T == 64) MR_FWD_ROW(64);
-    else if (T == 256) MR_FWD_ROW(256);
-    else MR_FWD_ROW(1024);
+    const int c = row_chunks(sh.gs, T);
+    if (T == 64 && c == 1) MR_FWD_ROW(64, 1);
+    else if (T == 64 && c == 2) MR_FWD_ROW(64, 2);
+    else if (T == 64) MR_FWD_ROW(64, 4);
+    else if (T == 256 && c == 2) MR_FWD_ROW(256, 2);
+    else if (T == 256) MR_FWD_ROW(256, 4);
+    else if (c == 2) MR_FWD_ROW(1024, 2);
+    else MR_FWD_ROW(1024, 4);
 #undef MR_FWD_ROW
   } else {
     const int64_t blocks = (sh.n_groups + 3) / 4;
@@ -1186,17 +1216,22 @@ int launch_bwd(const Shape& sh, const void* w, int wt, float* v, float* alpha, f
     else MR_BWD_FAST(MR_F32, MR_BF16);
 #undef MR_BWD_FAST_T
 #undef MR_BWD_FAST
-  } else if (sh.row && fast_align) {
+  } else if (sh.row && fast_align && row_backward(sh, MODE, wt)) {
     const int T = row_threads(sh.gs);
     const int64_t blocks = T == 64 ? (sh.n_groups + 3) / 4 : sh.n_groups;
     if (blocks > 0x7fffffff) return fail(MR_EINVAL, "mr_fq_backward_signsgd: tensor too large");
-#define MR_BWD_ROW(T_)                                                                                         \
-  hipLaunchKernelGGL((fq_bwd_row<MODE, UPDATE, T_>), dim3(static_cast<unsigned>(blocks)), dim3(T_ == 64 ? kBlock : T_), \
+#define MR_BWD_ROW(T_, C_)                                                                                     \
+  hipLaunchKernelGGL((fq_bwd_row<MODE, UPDATE, T_, C_>), dim3(static_cast<unsigned>(blocks)), dim3(T_ == 64 ? kBlock : T_), \
                      0, stream, w, wt, v, alpha, beta, init_scale, g, gt, sh.n_groups, sh.cols, sh.gs, sh.ng, sh.maxq, \
                      sh.inv_maxq, sh.qmin, sh.qmax, eps, st, gv_out, ga_out, gb_out, map)
-    if (T == 64) MR_BWD_ROW(64);
-    else if (T == 256) MR_BWD_ROW(256);
-    else MR_BWD_ROW(1024);
+    const int c = row_chunks(sh.gs, T);
+    if (T == 64 && c == 1) MR_BWD_ROW(64, 1);
+    else if (T == 64 && c == 2) MR_BWD_ROW(64, 2);
+    else if (T == 64) MR_BWD_ROW(64, 4);
+    else if (T == 256 && c == 2) MR_BWD_ROW(256, 2);
+    else if (T == 256) MR_BWD_ROW(256, 4);
+    else if (c == 2) MR_BWD_ROW(1024, 2);
+    else MR_BWD_ROW(1024, 4);
 #undef MR_BWD_ROW
   } else {
     const int64_t blocks = (sh.n_groups + 3) / 4;

@@ -335,3 +335,14 @@ def test_float16_output_is_the_narrowed_float32(mode, shape, wdtype):
                         for dt in (torch.float32, torch.float16))
         want = to_np(wide).astype(np.float16)
         assert np.array_equal(to_np(narrow).view(np.int16), want.view(np.int16))
+
+
+# The row kernels' other forms: one, two and four runs of 8 a thread of a wave
+# and four of 256 threads, full and one run past the form before; 8200 groups
+# of 264 leave the backward to the wave-per-group kernel.
+@pytest.mark.parametrize("mode", ["asym", "sym", "searched"])
+@pytest.mark.parametrize("shape", [(9, 264, -1), (9, 352, -1), (9, 504, -1), (9, 520, -1), (9, 1024, -1), (9, 1032, -1),
+                                   (5, 4096, -1), (5, 4104, -1), (3, 8192, -1), (3, 16384, -1), (3, 16392, -1), (8200, 264, -1)])
+@pytest.mark.parametrize("wdtype", [torch.bfloat16, torch.float32])
+def test_row_kernel_forms(mode, shape, wdtype):
+    test_long_groups_and_float16(mode, shape, wdtype)
