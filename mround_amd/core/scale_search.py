@@ -3,7 +3,7 @@
 Before the rounding is learned, a symmetric scheme below 4 bits picks each
 group's initial scale by trying a line of clipping thresholds and keeping
 the one with the least importance-weighted reconstruction error
-(``mr_search_scales``, one GPU thread per group). The searched scale then
+(``mr_search_scales``, one or more GPU lanes per group). The searched scale then
 enters fake quantization as ``init_scale`` with ``beta`` learning a factor
 around it (``ScaleInit.SEARCHED``).
 """

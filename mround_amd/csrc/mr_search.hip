@@ -16,9 +16,12 @@
 // Measured with importance on 11008 x 2048 bf16: groups of 64 at 2 bits (181
 // candidates) 725 us with a thread per group, 475 now (2.4 cycles an
 // instruction of a SIMD); groups of 128 at 3 bits 1260 -> 590; 192 x 576 at 2
-// bits 194 -> 9. (A min and max for the v_med3, or the rounding by adding and
-// taking off 1.5 * 2^23, measured 7-24 % slower. Ending a candidate when every
-// lane's partial sum exceeds its best saves 1-8 % of the elements: not done.)
+// bits 194 -> 9. Without importance groups of 64 fit six waves per SIMD
+// (18944 x 3584 at 3 bits 1832 -> 1561 us; a thread per group 1719, which at
+// groups of 128 takes 1836 to the 1867 here and at 192 x 576 190 to 10). (A min
+// and max for the v_med3, or the rounding by adding and taking off 1.5 * 2^23,
+// measured 7-24 % slower. Ending a candidate when every lane's partial sum
+// exceeds its best saves 1-8 % of the elements: not done.)
 //
 // Importance (the collecting forward of mround/pipeline/runner.py:346-363,
 // `sum(square(x), axis=0)` of each linear's input): per-column sums of
@@ -50,7 +53,7 @@ __device__ __forceinline__ int candidate(int o, int half) {
 }
 
 template <int GS, typename WT, bool IMP>
-__global__ __launch_bounds__(kBlock, GS == 32 ? 6 : GS == 64 ? 5 : 3) void search_kernel(const WT* __restrict__ w,
+__global__ __launch_bounds__(kBlock, GS == 32 || (GS == 64 && !IMP) ? 6 : GS == 64 ? 5 : 3) void search_kernel(const WT* __restrict__ w,
                                                         const float* __restrict__ imp,
                                                         int64_t rows, int groups_per_row,
                                                         int bits, double step, int half, int shift,
@@ -92,11 +95,17 @@ __global__ __launch_bounds__(kBlock, GS == 32 ? 6 : GS == 64 ? 5 : 3) void searc
   const float lo = -nmax, hi = nmax - 1.0f;
   const int count = 2 * half + 1;
 
+  // Short bfloat16 groups without importance count their loop in scalar
+  // registers (18944 x 3584 at 3 bits 1879 -> 1720 us; the other forms 1-4 % slower).
+  constexpr bool kCounted = GS == 32 && !IMP && sizeof(WT) == 2;
+  const int trips = (count + (1 << shift) - 1) >> shift;
+
   float best_s = 0.0f, best_l = __builtin_inff();
   int best_o = count;
   auto run = [&](auto fusedc) __attribute__((always_inline)) {
     constexpr bool FUSED = decltype(fusedc)::value;
-    for (int o = part; o < count; o += 1 << shift) {
+    for (int n = 0, o = part; kCounted ? n < trips : o < count; ++n, o += 1 << shift) {
+      if (kCounted && o >= count) break;
       const float eff = static_cast<float>(nmax_d - step * static_cast<double>(candidate(o, half)));
       const float inverse = (-eff) * recip;
       const float scale = inverse == 0.0f ? 0.0f : 1.0f / inverse;
