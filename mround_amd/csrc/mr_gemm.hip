@@ -114,7 +114,10 @@ __device__ __forceinline__ void tile_coords(int lt, int grid_m, int grid_n, int&
 // Block i of n, renumbered so that each XCD (blocks are dealt to the eight
 // round-robin) works through one contiguous run, whatever n. (Only multiples of
 // eight renumbered before: 16384 x 960 x 576 41 us on small tiles, 22 now;
-// 1024 x 3584 x 37888 298 -> 245.)
+// 1024 x 3584 x 37888 298 -> 245. With up to 8 k-tiles, where the outputs are most
+// of the bytes, other numbers stay in the order they are dealt: 532 small tiles
+// of 9728 x 896 x 256 13.2 us, renumbered 14.0, 3300 of 6968 x 7680 x 64 with
+// the SwiGLU 30.5 and 33.5.)
 __device__ __forceinline__ int xcd_order(int i, int n) {
   const int x = i & 7;
   return x * (n >> 3) + min(x, n & 7) + (i >> 3);
@@ -608,7 +611,7 @@ __global__ __launch_bounds__(kThreads) void gemm_kernel(GemmParams p) {
   if (p.ksplit > 1) {
     split = bid % p.ksplit;
     bid /= p.ksplit;
-  } else {
+  } else if ((p.n_tiles & 7) == 0 || p.K > 8 * BK) {
     bid = xcd_order(bid, p.n_tiles);
   }
   int bm, bn;
@@ -1379,28 +1382,36 @@ int split_plan(int64_t tiles, int KT, int64_t ws_bytes) {
 }
 
 // How a product runs is whichever of four plans the times below expect to take
-// least. The constants are microseconds, fitted to 304 products (the twelve of
-// a block over geometries of hidden 576 .. 3584 and 256 .. 8192 tokens, and the
-// vocabulary heads), each run by every plan, with its operands in cache and, for
-// half of them, from memory: median error 4-8 %, and the plan chosen is on
-// average 0.8 % slower than the best of them. The start and epilogue of a round
-// of tiles depend on the kind of output.
+// least, with the margins of plan_for. The constants are microseconds, fitted to
+// 304 products (the twelve of a block over geometries of hidden 576 .. 3584 and
+// 256 .. 8192 tokens, and the vocabulary heads), each run by every plan, with its
+// operands in cache and, for half of them, from memory, and the deep kernel's
+// slope over long runs to 667 from memory (those over 128 .. 8192 tokens, the
+// split-precision products and 120 of random sizes). Over these 667 the plan
+// chosen is on average 1.5 % slower than the best of the plans, and 10 % of them
+// and more slower than the large and small tiles alone for one (2560 x 2048 x
+// 4096 of MR_TN on 160 wide tiles, 59 -> 67; on average they gain 29 %). The start
+// and epilogue of a round of tiles depend on the kind of output.
 enum Output { OUT_B16, OUT_F32, OUT_RESID, OUT_SWIGLU, OUT_SWIGLU_BWD, OUTPUTS };
 
 // 128 x 128 or (wide) 256 x 128 tiles on the deep kernel, one block per CU:
 // rounds of 256, the tail past them cut along K into `split` blocks a tile, whose
 // partials take a round trip and a second kernel. A k-tile takes longer the more
-// CUs work.
+// CUs work, and, with operands from memory, `more` longer from the 25th of a run
+// on (128 x 128 tiles 0.6 us and more a k-tile: 1024 x 2560 x 6144 in one run 62
+// us, 49 on large tiles; of 46 such products with runs of 72 k-tiles and more 45
+// were slower than another plan, of 44 on wide tiles with runs of 120 and more 38).
 struct DeepTimes {
-  double launch, start[OUTPUTS], round, tail, busy, reduce, partial;
-  int max_kt;  // longest run of k-tiles the fit holds for (see kDeepMaxKtRounds)
+  double launch, start[OUTPUTS], round, tail, busy, reduce, partial, more;
 };
-constexpr DeepTimes kDeepTimes = {0.9, {3.0, 4.0, 5.4, 4.9, 6.7}, 0.453, 0.305, 0.149, 1.2, 0.035, 128};
-constexpr DeepTimes kWideTimes = {0.6, {4.3, 5.4, 7.5, 6.9, 11.0}, 0.838, 0.526, 0.266, 1.1, 0.051, 320};
+constexpr DeepTimes kDeepTimes = {0.9, {3.0, 4.0, 5.4, 4.9, 6.7}, 0.453, 0.305, 0.149, 1.2, 0.035, 0.15};
+constexpr DeepTimes kWideTimes = {0.6, {4.3, 5.4, 7.5, 6.9, 11.0}, 0.838, 0.526, 0.266, 1.1, 0.051, 0.06};
 double deep_time(const DeepTimes& c, int64_t tiles, int KT, int split, Output o) {
+  auto late = [&](int kt) { return kt > 24 ? c.more * (kt - 24) : 0.0; };
   const int64_t tail = tiles % 256, blocks = tail * split;
-  double t = c.launch + static_cast<double>(tiles / 256) * (c.start[o] + c.round * KT);
-  if (tail) t += c.start[o] + (KT + split - 1) / split * (c.tail + c.busy * static_cast<double>(blocks) / 256.0);
+  const int run = (KT + split - 1) / split;
+  double t = c.launch + static_cast<double>(tiles / 256) * (c.start[o] + c.round * KT + late(KT));
+  if (tail) t += c.start[o] + run * (c.tail + c.busy * static_cast<double>(blocks) / 256.0) + late(run);
   if (split > 1) t += c.reduce + c.partial * static_cast<double>(blocks);
   return t;
 }
@@ -1436,35 +1447,33 @@ struct Plan {
   int split;  // DEEP, WIDE: blocks per tail tile
 };
 
-// In longer runs than max_kt, or than this in whole rounds, the k-tile slows
-// beyond the fit when operands come from memory (128 x 128 tiles to 0.6 us:
-// 4096 x 896 x 9728 64 us from cache and 91 from memory, 95 inside a 0.5B block
-// step, against 69 and 83 on wide tiles cut in two, the step 693 -> 688;
-// 9728 x 896 x 16384, two whole rounds, 353 against 290 on large tiles; on wide
-// tiles 4096 x 2048 x 11008, one round, 148 and 177 against 160 and 170).
-constexpr int kDeepMaxKtRounds = 160;
-
 // The plan of an M x N x (64 KT) product with ws_bytes for partials. rows: M
 // counts activation rows (NT, NN), not weight rows (TN). There a product of
 // under kSplitMinKt k-tiles is never cut along K, so that a row's sums are the
 // same bits whatever other rows come with it: a step in pieces has the
 // activations of the whole batch's step. (Cutting them too gained 9 us of a
-// 0.5B scoring batch's 2,397.)
+// 0.5B scoring batch's 2,397.) The deep kernel is taken for 1.5 % or more, and of up
+// to kShortKt k-tiles large tiles over small ones for 12 % or more: within these
+// the times do not tell them apart, and the wrong one cost more than the right one
+// gave (weight gradients of 512 tokens and fewer, whose outputs are most of
+// their bytes: 3584 x 18944 x 512 100 us on small tiles, 108 on large).
+constexpr int kShortKt = 8;
 Plan plan_for(int64_t M, int64_t N, int KT, bool rows, Output o, int64_t ws_bytes) {
   const int64_t big = ((M + 255) / 256) * ((N + 255) / 256);
   const int64_t small = ((M + 127) / 128) * ((N + 127) / 128);
   const int64_t wide = ((M + 255) / 256) * ((N + 127) / 128);
   Plan p{BIG, 1};
   double best = big_time(big, KT, split_plan(big, KT, ws_bytes), o);
-  if (small_time(small, KT, o) < best) {
-    best = small_time(small, KT, o);
+  const double t_small = small_time(small, KT, o);
+  if (t_small * (KT <= kShortKt ? 0.88 : 1.0) < best) {
+    best = t_small;
     p.kind = SMALL;
   }
+  best *= 0.985;
   auto deep = [&](Kind kind, const DeepTimes& times, int64_t tiles, int64_t tile_bytes) {
     const int64_t tail = tiles % 256;
     for (int sp = 1; sp <= 16; ++sp) {
       if (sp > 1 && (!tail || (rows && KT < kSplitMinKt) || tail * sp > 256 || sp * 2 > KT || tail * sp * tile_bytes > ws_bytes)) break;
-      if ((KT + sp - 1) / sp > times.max_kt || (tiles >= 256 && KT > kDeepMaxKtRounds)) continue;
       const double t = deep_time(times, tiles, KT, sp, o);
       if (t < best) {
         best = t;
