@@ -296,6 +296,18 @@ int mr_embed_rows(const void* table, int dtype, int64_t V, int64_t H, int64_t ld
  */
 enum { MR_NT = 0, MR_NN = 1, MR_TN = 2 };
 size_t mr_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
+
+/*
+ * The plan of such a product (N its width, as above) with workspace_bytes for
+ * partials, without launching it: the tiles it runs on (256 x 256, with or
+ * without its last wave as quarter tiles; 128 x 128 two to a CU; deep-pipelined
+ * 128 x 128 or 256 x 128), the blocks along K of each tile past the whole waves
+ * of 256 (1: not cut), and how many such tiles there are.
+ */
+enum { MR_OUT_F32 = 0, MR_OUT_BF16 = 1, MR_OUT_RESID = 2, MR_OUT_SWIGLU = 3, MR_OUT_SWIGLU_SPLIT = 4, MR_OUT_SWIGLU_BWD = 5 };
+enum { MR_TILES_LARGE = 0, MR_TILES_LARGE_QUARTERS = 1, MR_TILES_SMALL = 2, MR_TILES_DEEP = 3, MR_TILES_WIDE = 4 };
+int mr_gemm_plan(int layout, int output, int64_t M, int64_t N, int64_t K, size_t workspace_bytes, int* tiles_out,
+                 int* split_out, int64_t* tail_out);
 int mr_gemm(int layout, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda,
             const void* B, int64_t ldb, void* C, int c_dtype, int64_t ldc, const float* bias,
             const float* resid, int64_t ldr, void* workspace, size_t workspace_bytes,

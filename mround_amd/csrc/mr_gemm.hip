@@ -1512,6 +1512,9 @@ int64_t split_bytes(int64_t M, int64_t N, int64_t K) {
   return bytes;
 }
 
+// Whether the last wave of a large-tile launch runs as quarter tiles (see launch).
+bool quarter_tail(int64_t tiles, int split) { return split == 1 && tiles >= 256 && tiles % 256 && tiles % 256 <= 128; }
+
 // Large tiles go out in whole waves of 256 (one per CU). When K is long (at
 // least kSplitMinKt steps, so a tile takes far longer than the partial-tile
 // round trip), a remainder that would leave CUs idle in a last, partial wave
@@ -1558,7 +1561,7 @@ int launch(GemmParams p, hipStream_t s) {
     // the 7B block's q/k/v projection (4.5 waves) and its attention-output and
     // q/k/v input gradients (3.5 waves). (The residual and SwiGLU-backward
     // epilogues ran no faster or slower on quarter tiles.)
-    if (split == 1 && full && tail && tail <= wave / 2) {
+    if (quarter_tail(tiles, split)) {
       launch_whole<AK, BKM, EPI, OB>(p, 0, full, s);
       GemmParams q = p;
       q.ksplit = 1;
@@ -1756,6 +1759,31 @@ extern "C" {
 size_t mr_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   return static_cast<size_t>(mr::split_bytes(M, N, K));
+}
+
+int mr_gemm_plan(int layout, int output, int64_t M, int64_t N, int64_t K, size_t workspace_bytes, int* tiles_out,
+                 int* split_out, int64_t* tail_out) {
+  using namespace mr;
+  clear_error();
+  if (layout < 0 || layout > 2 || output < MR_OUT_F32 || output > MR_OUT_SWIGLU_BWD)
+    return fail(MR_EINVAL, "mr_gemm_plan: unknown layout %d or output %d", layout, output);
+  if (M <= 0 || N <= 0 || K <= 0 || K % BK || M > 0x7fffffff || N > 0x7fffffff || K > 0x7fffffff)
+    return fail(MR_EINVAL, "mr_gemm_plan: M and N positive, K a positive multiple of %d", BK);
+  if (!tiles_out || !split_out || !tail_out) return fail(MR_EINVAL, "mr_gemm_plan: null output");
+  constexpr Output kinds[] = {OUT_F32, OUT_B16, OUT_RESID, OUT_SWIGLU, OUT_F32, OUT_SWIGLU_BWD};
+  const int KT = static_cast<int>(K / BK);
+  const int64_t ws = static_cast<int64_t>(workspace_bytes < kSplitCapBytes ? workspace_bytes : kSplitCapBytes);
+  const Plan p = plan_for(M, N, KT, layout != MR_TN, kinds[output], ws);
+  const int64_t bm = p.kind == BIG || p.kind == WIDE ? 256 : 128, bn = p.kind == BIG ? 256 : 128;
+  const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+  int split = p.kind == BIG ? split_plan(tiles, KT, ws) : p.split;
+  if (p.kind != SMALL && split > 1) split = (KT + (KT + split - 1) / split - 1) / ((KT + split - 1) / split);  // no empty split
+  const bool quarters = p.kind == BIG && (output <= MR_OUT_BF16 || output == MR_OUT_SWIGLU_SPLIT) && quarter_tail(tiles, split);
+  *tiles_out = p.kind == BIG ? (quarters ? MR_TILES_LARGE_QUARTERS : MR_TILES_LARGE)
+                             : p.kind == SMALL ? MR_TILES_SMALL : p.kind == DEEP ? MR_TILES_DEEP : MR_TILES_WIDE;
+  *split_out = split;
+  *tail_out = p.kind == SMALL ? tiles : tiles % 256;
+  return MR_OK;
 }
 
 int mr_gemm(int layout, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda,

@@ -78,6 +78,7 @@ _SIGNATURES = {
     "mr_delta_loss": (_I, [_P, _I, _P, _L, _L, _I, _P, _I, _I, _F, _P, _P, _P]),
     "mr_copy_bytes": (_I, [_P, _P, ctypes.c_size_t, _P]),
     "mr_gemm_workspace_bytes": (ctypes.c_size_t, [_L, _L, _L]),
+    "mr_gemm_plan": (_I, [_I, _I, _L, _L, _L, ctypes.c_size_t, _P, _P, _P]),
     "mr_gemm": (_I, [_I, _L, _L, _L, _P, _L, _P, _L, _P, _I, _L, _P, _P, _L, _P, ctypes.c_size_t, _P]),
     "mr_gemm_f32": (_I, [_I, _L, _L, _L, _P, _L, _P, _P, _L, _P, _L, _P]),
     "mr_gemm_f32_workspace_bytes": (ctypes.c_size_t, [_L, _L, _L]),
@@ -410,6 +411,22 @@ def gemm_workspace_bytes(M: int, N: int, K: int) -> int:
     """``mr_gemm_workspace_bytes``: k-split partials for an M x N x K product
     (N is the product's width: 2N for the SwiGLU pair)."""
     return int(lib().mr_gemm_workspace_bytes(M, N, K))
+
+
+GEMM_OUTPUT = {"f32": 0, "bf16": 1, "resid": 2, "swiglu": 3, "swiglu_split": 4, "swiglu_bwd": 5}
+GEMM_TILES = ("large", "large_quarters", "small", "deep", "wide")
+
+
+def gemm_plan(layout: str, output: str, M: int, N: int, K: int, workspace_bytes: int | None = None) -> tuple[str, int, int]:
+    """``mr_gemm_plan``: (tiles, blocks along K of a tail tile, tail tiles) of a
+    product of width N, with ``workspace_bytes`` for partials (None: what
+    ``gemm_workspace_bytes`` asks for)."""
+    ws = gemm_workspace_bytes(M, N, K) if workspace_bytes is None else workspace_bytes
+    tiles, split, tail = ctypes.c_int(), ctypes.c_int(), ctypes.c_int64()
+    rc = lib().mr_gemm_plan(GEMM_LAYOUT[layout], GEMM_OUTPUT[output], M, N, K, ws, ctypes.byref(tiles),
+                            ctypes.byref(split), ctypes.byref(tail))
+    _check(rc, "mr_gemm_plan")
+    return GEMM_TILES[tiles.value], split.value, tail.value
 
 
 def _gemm_ws(device: torch.device, M: int, N: int, K: int, workspace):

@@ -167,6 +167,31 @@ def test_gemm_workspace_unsplit_shapes(lib, M, N, K):
     assert lib.mr_gemm_workspace_bytes(M, N, K) == 0
 
 
+def test_gemm_plan(lib):
+    from mround_amd import kernels as K
+
+    # whole waves of large tiles; a last half wave as quarter tiles (of a plain
+    # output); a long K cut along it, and not without a workspace
+    assert K.gemm_plan("nt", "bf16", 16384, 4096, 18944) == ("large", 1, 0)
+    assert K.gemm_plan("nt", "f32", 16384, 4608, 3584) == ("large_quarters", 1, 128)
+    assert K.gemm_plan("nt", "resid", 16384, 4608, 3584) == ("large", 1, 128)
+    tiles, split, tail = K.gemm_plan("tn", "f32", 576, 576, 4096)
+    assert tiles == "deep" and tail == 25
+    assert 1 < split and K.gemm_workspace_bytes(576, 576, 4096) >= tail * split * 128 * 128 * 4
+    assert K.gemm_plan("tn", "f32", 576, 576, 4096, workspace_bytes=0) == ("deep", 1, 25)
+    # activation rows of a short K are never cut
+    for m in (8, 128, 1000, 4096, 16384):
+        for n in (64, 896, 4864, 37888):
+            for k in (64, 896, 3584, 6080):
+                for lay, out in (("nt", "f32"), ("nn", "bf16"), ("nt", "resid"), ("nt", "swiglu"), ("nn", "swiglu_bwd")):
+                    assert K.gemm_plan(lay, out, m, n, k)[1] == 1
+    i, t = ctypes.c_int(), ctypes.c_int64()
+    out = ctypes.byref(i), ctypes.byref(i), ctypes.byref(t)
+    for bad in ((3, 0, 64, 64, 64), (0, 6, 64, 64, 64), (0, 0, 0, 64, 64), (0, 0, 64, 64, 65)):
+        assert lib.mr_gemm_plan(*bad, 0, *out) == -22
+        assert b"mr_gemm_plan" in lib.mr_last_error()
+
+
 def test_gemm_calls_share_no_workspace(lib):
     # a weight gradient of short K, cut along K: without a workspace each call
     # has partials of its own, so that calls on two streams do not meet in them

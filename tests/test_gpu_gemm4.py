@@ -148,10 +148,10 @@ def test_4wave_swiglu_backward(kt):
 @pytest.mark.parametrize("layout", ["nt", "nn", "tn"])
 @pytest.mark.parametrize("mnk", [(4096, 4352, 6144), (904, 696, 6400)])
 def test_4wave_k_split(layout, mnk):
-    # 4096 x 4352: one whole wave of 256 tiles and 16 past it, cut along K;
-    # 904 x 696 (12 tiles, under one wave, long K): the whole grid cut along K.
-    # The split blocks run on the 4-wave kernel and write raw partial tiles
-    # that the reduce kernel sums in split order, as the 8-wave kernel's do.
+    # 4096 x 4352: one whole wave of 256 large tiles and 16 past it, cut along
+    # K; 904 x 696 (under one wave, long K): the whole grid cut along K, on deep
+    # tiles (large ones in test_planned). The split blocks write raw partial
+    # tiles that the reduce kernel sums in split order, as the 8-wave kernel's do.
     M, N, Kd = mnk
     print("case gemm4 k-split", layout, mnk, flush=True, file=sys.stderr)
     a, b, a_ref, b_ref = _operands(layout, M, N, Kd, seed=170)
@@ -167,12 +167,12 @@ def test_4wave_k_split(layout, mnk):
     assert torch.equal(c, c8), "4-wave and 8-wave kernels differ"
 
 
-# The deep 128 x 128 kernel (four LDS stages) on small grids: every entry
-# position into the stage pattern and K shorter than it (KT = 1 .. 9), ragged
-# edges, a grid past one round whose tail is cut along K (258 tiles), and
-# k-split grids with every epilogue, against a float32 product within the
-# accumulation bound and bit for bit against the 8-wave kernel on the same
-# tiles and splits.
+# Small grids: the double-buffered small tiles (KT = 1 .. 5, by output), the deep
+# 128 x 128 kernel (four LDS stages) past them and on k-split grids with every
+# epilogue, ragged edges, and 5504 x 760 on wide or small tiles, against a
+# float32 product within the accumulation bound and bit for bit against the
+# 8-wave kernel on the same tiles and splits (small tiles run there as they are).
+# test_planned holds the plans.
 @pytest.mark.parametrize("layout", ["nt", "nn", "tn"])
 @pytest.mark.parametrize("mnk", [(264, 328, 64 * kt) for kt in (1, 2, 3, 4, 5, 9)]
                          + [(128, 128, 6144), (584, 568, 6208), (5504, 760, 1280)])
@@ -287,3 +287,42 @@ def test_wide_swiglu(kt):
         outs.append((act, gu, dgu))
     assert all(torch.equal(a, b) for a, b in zip(*outs)), "the wide and 8-wave kernels differ"
     assert bool(torch.all((outs[0][1].float() - gu_ref).abs() <= bound + gu_ref.abs() * 2.0**-8))
+
+
+# The wide SwiGLU forms at each phase of the three-stage pattern, and the deep
+# backward (one that takes the deep kernel from its first k-tile) at K about the
+# length of its four stages.
+@pytest.mark.parametrize("kt", [24, 25, 26])
+def test_wide_swiglu_phases(kt):
+    assert K.gemm_plan("nt", "swiglu", 2056, 2 * 1568, 64 * kt)[0] == "wide"
+    assert K.gemm_plan("nn", "swiglu_bwd", 2056, 3072, 64 * kt)[0] == "wide"
+    test_wide_swiglu(kt)
+
+
+@pytest.mark.parametrize("kd", [64, 128, 192, 256, 320])
+def test_deep_swiglu_short(kd):
+    assert K.gemm_plan("nn", "swiglu_bwd", 392, 352, kd)[0] == "deep"
+    test_deep_swiglu(kd)
+
+
+# Each kind of plan, named: (tiles, blocks along K of a tail tile, tail tiles).
+# Deep runs of 2 and 3 k-tiles and a last run of 1; deep, wide and large grids
+# past one round with the tail cut; large grids under one round cut; the phases
+# of the deep (KT % 4) and wide (KT % 3) patterns.
+@pytest.mark.parametrize(("plan", "layouts", "kind", "mnk"), [
+    (("deep", 4, 2), "tn", "f32", (136, 72, 512)), (("deep", 3, 2), "tn", "resid", (136, 72, 576)),
+    (("deep", 5, 2), "tn", "f32", (136, 72, 832)), (("deep", 1, 9), "nt nn tn", "resid", (264, 328, 384)),
+    (("deep", 1, 9), "nt nn tn", "f32", (264, 328, 448)), (("deep", 1, 9), "nt nn tn", "bf16 bias", (264, 328, 512)),
+    (("deep", 1, 9), "nt nn tn", "f32", (264, 328, 576)), (("deep", 8, 4), "tn", "bf16 bias", (584, 6632, 1536)),
+    (("deep", 16, 4), "nt nn", "f32", (584, 6632, 6144)), (("deep", 16, 4), "nt", "resid", (584, 6632, 6144)),
+    (("wide", 7, 30), "nt nn tn", "f32", (5384, 1544, 6208)), (("wide", 1, 225), "nt nn tn", "f32", (2056, 3080, 1536)),
+    (("wide", 1, 225), "nt nn tn", "bf16 bias", (2056, 3080, 1600)),
+    (("wide", 1, 225), "nt nn tn", "resid", (2056, 3080, 1664)),
+    (("large", 5, 48), "nt nn", "f32", (712, 4072, 6144)), (("large", 5, 48), "tn", "resid", (712, 4072, 6208)),
+    (("large", 16, 16), "nt nn tn", "f32", (4096, 4352, 6144)),
+    (("small", 1, 9), "nt nn tn", "bf16 bias", (264, 328, 64)), (("small", 1, 9), "nt nn tn", "resid", (264, 328, 192)),
+])
+def test_planned(plan, layouts, kind, mnk):
+    for layout in layouts.split():
+        assert K.gemm_plan(layout, {"bf16 bias": "bf16"}.get(kind, kind), *mnk) == plan
+        test_deep(layout, mnk, kind)

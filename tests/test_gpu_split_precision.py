@@ -485,8 +485,8 @@ def test_search_weighs_what_the_forward_wrote(split):
         assert bool(torch.isfinite(got).all()) and differ <= 2e-3, n
 
 
-# Ragged tiles, a tail cut along K (K 6144 and up) on the deep and the large
-# tiles, and whole rounds of large tiles.
+# Ragged small tiles, the deep kernel whole and cut along K (K 6144), large tiles
+# uncut, and many rounds of small ones; the other plans below.
 @pytest.mark.parametrize(("M", "N", "Kd"), [(8, 32, 64), (136, 96, 192), (264, 1536, 1728), (904, 352, 6144),
                                             (512, 11008, 6144), (2048, 8576, 448)])
 @pytest.mark.parametrize("save", [True, False])
@@ -509,3 +509,16 @@ def test_swiglu_split_epilogue(M, N, Kd, save):
     if save:
         assert torch.equal(act.view(torch.int16), want.view(torch.int16))
         assert torch.equal(gu.view(torch.int16), want_gu.view(torch.int16))
+
+
+# The split epilogue on each kind of tiles that its plans reach: wide ones at each
+# phase of their pattern, large ones with a last wave of quarter tiles, and large
+# and deep ones cut along K.
+@pytest.mark.parametrize(("plan", "M", "N", "Kd"), [
+    (("wide", 1, 130), 1224, 1632, 1152), (("wide", 1, 130), 1224, 1632, 1600), (("wide", 1, 130), 1224, 1632, 1664),
+    (("large_quarters", 1, 89), 5832, 1888, 768), (("large", 5, 48), 6088, 224, 6144),
+    (("large", 16, 3), 9416, 864, 6144), (("deep", 4, 48), 904, 352, 6144)])
+@pytest.mark.parametrize("save", [True, False])
+def test_swiglu_split_plans(plan, M, N, Kd, save):
+    assert K.gemm_plan("nt", "swiglu_split", M, 2 * N, Kd) == plan
+    test_swiglu_split_epilogue(M, N, Kd, save)
