@@ -175,7 +175,11 @@ struct Share {
   }
 };
 
-// The tile by the fp32 MFMA over k in [k_lo, k_hi).
+// The tile by the fp32 MFMA over k in [k_lo, k_hi), the next k tile's loads in
+// flight during this one's MFMAs. (Loaded and multiplied in turn, it took two to
+// three times as long: 4096 x 3584 x 3584 with such a value in every block 4400
+// us, 1980 here, 1250-1580 on the fp32 MFMA alone; 896 x 4864 x 1000 375, 200 and
+// 190-240; 1000 x 896 x 4864 less B2 490, 380 and 1240.)
 template <bool A_KMAJOR, bool B_KMAJOR>
 __device__ __forceinline__ void tile_fp32(const Operand& A, const Operand& B, int m0, int n0, int k_lo, int k_hi,
                                           uint8_t* lds, f32x16 (&acc)[2][2]) {
@@ -187,16 +191,36 @@ __device__ __forceinline__ void tile_fp32(const Operand& A, const Operand& B, in
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = f32x16{};
-  for (int k0 = k_lo; k0 < k_hi; k0 += TK) {
-    __syncthreads();
+  float ra[PER], rb[PER];
+  auto slot = [](int i, bool kmajor, int& r, int& k) __attribute__((always_inline)) {
+    const int idx = i * kThreads + static_cast<int>(threadIdx.x);
+    r = kmajor ? idx / TK : idx % TM;
+    k = kmajor ? idx % TK : idx / TM;
+  };
+  auto load = [&](int k0) __attribute__((always_inline)) {
+#pragma unroll
     for (int i = 0; i < PER; ++i) {
-      const int idx = i * kThreads + static_cast<int>(threadIdx.x);
-      const int ka = A_KMAJOR ? idx % TK : idx / TM, ra = A_KMAJOR ? idx / TK : idx % TM;
-      const int kb = B_KMAJOR ? idx % TK : idx / TN, rb = B_KMAJOR ? idx / TK : idx % TN;
-      As[ka][ra] = at<A_KMAJOR>(A, m0 + ra, k0 + ka, k_hi);
-      Bs[kb][rb] = at<B_KMAJOR>(B, n0 + rb, k0 + kb, k_hi);
+      int r, k;
+      slot(i, A_KMAJOR, r, k);
+      ra[i] = at<A_KMAJOR>(A, m0 + r, k0 + k, k_hi);
+      slot(i, B_KMAJOR, r, k);
+      rb[i] = at<B_KMAJOR>(B, n0 + r, k0 + k, k_hi);
+    }
+  };
+  load(k_lo);
+  for (int k0 = k_lo; k0 < k_hi; k0 += TK) {
+    __syncthreads();  // every read of the previous tile (or of the planes) is done
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      int r, k;
+      slot(i, A_KMAJOR, r, k);
+      As[k][r] = ra[i];
+      slot(i, B_KMAJOR, r, k);
+      Bs[k][r] = rb[i];
     }
     __syncthreads();
+    if (k0 + TK < k_hi) load(k0 + TK);
+#pragma unroll
     for (int kk = 0; kk < TK; kk += 2) {
       float a[2], b[2];
 #pragma unroll
