@@ -145,7 +145,8 @@ __device__ __forceinline__ int swz_bits(int row) { return (row >> 1) & 7; }
 // rows or columns that are never stored.
 // Buffer resource over `bytes` bytes from `base`. Every offset the loads use
 // is already clamped inside the operand (see the loaders), so the resource
-// bound is only a second fence.
+// bound is only a second fence (the deep kernel, whose base moves along K,
+// sets none).
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 constexpr int kRsrcFlags = 0x00020000;  // raw 32-bit dwords, no swizzle
 __device__ __forceinline__ rsrc_t make_rsrc(const void* base, int64_t bytes) {
