@@ -322,7 +322,8 @@ int mr_gemm(int layout, int64_t M, int64_t N, int64_t K, const void* A, int64_t 
  * loop, the layer residual x (W' - W)^T and the weight gradient
  * (dL/dr)^T x (mround/core/tuning.py:140-190). The _ws form takes a workspace
  * for the k-split partials of a grid that would leave CUs idle (16-byte
- * aligned; a smaller or NULL one drops the split).
+ * aligned, apart from A, B, B2 and C, refused with MR_EINVAL otherwise; a
+ * smaller or NULL one drops the split).
  */
 size_t mr_gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int mr_gemm_f32_ws(int layout, int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, const float* B,

@@ -518,6 +518,14 @@ int mr_gemm_f32_ws(int layout, int64_t M, int64_t N, int64_t K, const float* A, 
   p.full = static_cast<int>(tiles - p.tail);
   int sp = workspace ? split_plan(p.tail, KT) : 1;
   if (static_cast<size_t>(p.tail) * sp * TM * TN * 4 > workspace_bytes) sp = 1;
+  if (sp > 1) {  // tiles read operand panels while others write their partials
+    const int64_t n = static_cast<int64_t>(p.tail) * sp * TM * TN * 4;
+    auto span = [](int64_t rows, int64_t ld, int64_t width) { return ((rows - 1) * ld + width) * 4; };
+    const int64_t a = a_kmajor ? span(M, lda, K) : span(K, lda, M), b = b_kmajor ? span(N, ldb, K) : span(K, ldb, N);
+    if (overlap(workspace, n, A, a) || overlap(workspace, n, B, b) || (B2 && overlap(workspace, n, B2, b)) ||
+        overlap(workspace, n, C, span(M, ldc, N)))
+      return fail(MR_EINVAL, "mr_gemm_f32: the workspace must not overlap A, B, B2 or C");
+  }
   const int64_t per = KT ? (KT + sp - 1) / sp : 0;
   p.kt_per = static_cast<int>(per);
   p.ksplit = per ? static_cast<int>((KT + per - 1) / per) : 1;  // no empty split

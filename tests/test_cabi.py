@@ -167,6 +167,20 @@ def test_gemm_workspace_unsplit_shapes(lib, M, N, K):
     assert lib.mr_gemm_workspace_bytes(M, N, K) == 0
 
 
+def test_gemm_f32_refuses_a_workspace_over_its_operands(lib):
+    P = ctypes.c_void_p
+    M, N, K = 256, 128, 4096  # two tiles, cut along K
+    nbytes = lib.mr_gemm_f32_workspace_bytes(M, N, K)
+    assert nbytes > 0
+    a, b, b2, c = (k << 30 for k in (1, 2, 3, 4))
+    for layout in (0, 1, 2):
+        lda, ldb = (K if layout != 2 else M), (K if layout == 0 else N)
+        # at each operand's start, and reaching into it from before its first byte
+        for ws in (a, b, b2, c, a + M * K * 4 - 16, c - nbytes + 16):
+            rc = lib.mr_gemm_f32_ws(layout, M, N, K, P(a), lda, P(b), P(b2), ldb, P(c), N, P(ws), nbytes, None)
+            assert rc == -22 and b"overlap" in lib.mr_last_error()
+
+
 def test_gemm_plan(lib):
     from mround_amd import kernels as K
 
